@@ -15,6 +15,10 @@ magma_int_t getrf_batched_async(int m, int n, double** dA_array, int ldda, int**
 {
     if (m == n && getrf_tile_supported(n))
         return getrf_tile_launch(n, dA_array, ldda, ipiv_array, info_array, batch, stream);
+    if (getrf_wg_preferred(m, n, batch)) {
+        SizeArgs sz{m, n, ldda, nullptr, nullptr, nullptr, nullptr};
+        return getrf_wg_launch(sz, m, dA_array, ipiv_array, info_array, WgRhs<double>{}, batch, stream);
+    }
     if (getrf_lds_bytes(m, n) <= max_dynamic_lds())
         return getrf_lds_launch(m, n, dA_array, ldda, ipiv_array, info_array, batch, stream);
     if (getrf_blocked_supported(m))
@@ -117,6 +121,14 @@ magma_int_t magma_dgesv_batched(magma_int_t n, magma_int_t nrhs, double** dA_arr
     if (mgi::gesv_tile_supported(n, nrhs))
         return mgi::gesv_tile_launch(n, nrhs, dA_array, ldda, dipiv_array, dinfo_array, dB_array, lddb,
                                      batchCount, queue->stream);
+    if (mgi::getrf_wg_preferred(n, n, batchCount) && nrhs <= 16) {
+        mgi::SizeArgs sz{n, n, ldda, nullptr, nullptr, nullptr, nullptr};
+        mgi::WgRhs<double> rhs;
+        rhs.dB_array = dB_array;
+        rhs.nrhs = rhs.max_nrhs = nrhs;
+        rhs.lddb = lddb;
+        return mgi::getrf_wg_launch(sz, n, dA_array, dipiv_array, dinfo_array, rhs, batchCount, queue->stream);
+    }
     info = mgi::getrf_batched_async(n, n, dA_array, ldda, dipiv_array, dinfo_array, batchCount, queue->stream);
     if (info != MAGMA_SUCCESS) return info;
     return mgi::getrs_batched_async(0, n, nrhs, dA_array, ldda, dipiv_array, dB_array, lddb,
@@ -166,6 +178,10 @@ namespace mgi {
 magma_int_t sgetrf_batched_async(int m, int n, float** dA_array, int ldda, int** ipiv_array, int* info_array,
                                  int batch, hipStream_t stream)
 {
+    if (getrf_wg_preferred(m, n, batch)) {
+        SizeArgs sz{m, n, ldda, nullptr, nullptr, nullptr, nullptr};
+        return sgetrf_wg_launch(kUpdF32, sz, m, dA_array, ipiv_array, info_array, WgRhs<float>{}, batch, stream);
+    }
     if (getrf_lds_bytes(m, n, sizeof(float)) <= max_dynamic_lds())
         return sgetrf_lds_launch(m, n, dA_array, ldda, ipiv_array, info_array, batch, stream);
     if (getrf_blocked_supported(m))

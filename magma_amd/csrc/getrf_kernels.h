@@ -87,6 +87,25 @@ magma_int_t sgetrf_blocked_launch(int mode, int m, int n, int ldda, const int* m
                                   const int* ld_arr, int max_m, int max_n, float** dA_array, int** ipiv_array,
                                   int* info_array, int batch, hipStream_t stream);
 
+// getrf_wg.hip: one workgroup per system, at most 512 rows (any columns),
+// with up to 32 right-hand sides carried along and solved (dB_array not null;
+// square systems).
+template <typename T>
+struct WgRhs {
+    T** dB_array = nullptr;
+    int nrhs = 0, lddb = 0, max_nrhs = 0;
+    const int* nrhs_arr = nullptr;
+    const int* lddb_arr = nullptr;
+};
+bool getrf_wg_supported(int max_m);
+// Whether the one-workgroup kernel is the faster choice for a batch of m x n
+// systems (the rule's reasons are at its definition).
+bool getrf_wg_preferred(int max_m, int max_n, int batch);
+magma_int_t getrf_wg_launch(const SizeArgs& sz, int max_m, double** dA_array, int** ipiv_array, int* info_array,
+                            const WgRhs<double>& rhs, int batch, hipStream_t stream);
+magma_int_t sgetrf_wg_launch(int mode, const SizeArgs& sz, int max_m, float** dA_array, int** ipiv_array,
+                             int* info_array, const WgRhs<float>& rhs, int batch, hipStream_t stream);
+
 // Per-matrix arguments of the tile kernels (fixed size when arrays are null;
 // `map` sends workgroup b to matrix map[b]).
 struct TileArgs {

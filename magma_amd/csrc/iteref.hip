@@ -577,8 +577,13 @@ magma_int_t iteref_batched(int trans, int n, int nrhs, double** dA_array, int ld
     ir_lag2s_kernel<<<batch, kIrThreads, 0, stream>>>(n, dA_array, ldda, As, st.fail, anrm, lu_n);
     MGI_LAUNCH_CHECK();
     // 2. low-precision LU of the systems whose down-cast stayed finite
-    magma_int_t rc = sgetrf_blocked_launch(mode, n, n, n, lu_n, lu_n, nullptr, n, n, As_ptr, ipiv_ptr, lp_info,
-                                           batch, stream);
+    magma_int_t rc;
+    if (getrf_wg_preferred(n, n, batch)) {
+        const SizeArgs sz{n, n, n, lu_n, lu_n, nullptr, nullptr};
+        rc = sgetrf_wg_launch(mode, sz, n, As_ptr, ipiv_ptr, lp_info, WgRhs<float>{}, batch, stream);
+    } else {
+        rc = sgetrf_blocked_launch(mode, n, n, n, lu_n, lu_n, nullptr, n, n, As_ptr, ipiv_ptr, lp_info, batch, stream);
+    }
     if (rc != MAGMA_SUCCESS) return rc;
     ir_check_lu_kernel<<<batch, kIrThreads, 0, stream>>>(n, As, lp_info, st.fail);
     MGI_LAUNCH_CHECK();
@@ -689,7 +694,10 @@ magma_int_t iteref_batched(int trans, int n, int nrhs, double** dA_array, int ld
             frc = getrf_tile_launch_args((n + 15) / 16, a, dA_array, d_ipiv64_ptr, info_out, nf, stream);
         } else {
             SizeArgs sz{n, n, ldda, nullptr, nullptr, nullptr, d_map};
-            frc = getrf_blocked_launch_sz(sz, n, n, dA_array, d_ipiv64_ptr, info_out, nf, stream);
+            if (getrf_wg_preferred(n, n, nf))
+                frc = getrf_wg_launch(sz, n, dA_array, d_ipiv64_ptr, info_out, WgRhs<double>{}, nf, stream);
+            else
+                frc = getrf_blocked_launch_sz(sz, n, n, dA_array, d_ipiv64_ptr, info_out, nf, stream);
         }
         if (frc == MAGMA_SUCCESS) {
             // X = B for the fallback systems, then solve in place

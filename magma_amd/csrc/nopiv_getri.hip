@@ -104,6 +104,10 @@ void make_butterfly(int n2, std::vector<double>& u, std::vector<double>& v, unsi
 magma_int_t nopiv_getrf_async(int m, int n, double** dA_array, int ldda, const int* m_arr, const int* n_arr,
                               const int* ld_arr, int max_m, int max_n, int* info_array, int batch, hipStream_t st)
 {
+    if (getrf_wg_preferred(max_m, max_n, batch)) {
+        SizeArgs sz{m, n, ldda, m_arr, n_arr, ld_arr, nullptr};
+        return getrf_wg_launch(sz, max_m, dA_array, nullptr, info_array, WgRhs<double>{}, batch, st);
+    }
     if (!getrf_blocked_supported(max_m)) return MAGMA_ERR_NOT_SUPPORTED;
     return getrf_blocked_launch(m, n, ldda, m_arr, n_arr, ld_arr, max_m, max_n, dA_array, nullptr, info_array,
                                 batch, st);

@@ -7,6 +7,8 @@
 // n-buckets:
 //   * square n <= 128: the register-tile kernel instance for ceil(n/16)
 //     (fused with the solve when nrhs <= 16);
+//   * up to 512 rows: the one-workgroup kernel, the solve included when nrhs
+//     <= 16;
 //   * larger or rectangular: the blocked path with a panel width per bucket,
 // each bucket launched over an index map of its members. A plan holds the
 // buckets and their device maps, so executing it allocates nothing, does not
@@ -55,7 +57,10 @@ struct VBucket {
     int offset;      // into the concatenated map
 };
 
-enum VbVariant { kVbAuto = 0, kVbTile = 1, kVbBlocked32 = 2, kVbBlocked16 = 3, kVbBlocked8 = 4, kVbBlocked2x32 = 5 };
+enum VbVariant {
+    kVbAuto = 0, kVbTile = 1, kVbBlocked32 = 2, kVbBlocked16 = 3, kVbBlocked8 = 4, kVbBlocked2x32 = 5,
+    kVbWg = 6,               // one workgroup per system (n <= 512)
+};
 
 // panel width of a blocked variant (64 = the two-level form)
 static int variant_nb(int v)
@@ -101,8 +106,10 @@ static bool build_buckets(const int* h_m, const int* h_n, const int* h_nrhs, int
         int v = (variants && vb.id >= 0) ? variants[vb.id] : kVbAuto;
         const bool tile_ok = vb.id >= 0 && vb.max_n <= 128 && (!solve || vb.max_nrhs <= 16);
         if (v == kVbTile && !tile_ok) v = kVbAuto;
+        if (v == kVbWg && !getrf_wg_supported(vb.max_m)) v = kVbAuto;
         if (variant_nb(v) != 0 && !blocked_nb_valid(vb.max_m, variant_nb(v))) v = kVbAuto;
-        if (v == kVbAuto) v = tile_ok ? kVbTile : kVbBlocked32;
+        if (v == kVbAuto)
+            v = tile_ok ? kVbTile : getrf_wg_preferred(vb.max_m, vb.max_n, vb.count) ? kVbWg : kVbBlocked32;
         if (variant_nb(v) != 0 && !blocked_nb_valid(vb.max_m, variant_nb(v))) {
             v = blocked_nb_valid(vb.max_m, 16) ? kVbBlocked16 : kVbBlocked8;
         }
@@ -146,9 +153,22 @@ static magma_int_t exec_buckets(const std::vector<VBucket>& buckets, const int* 
                        : getrf_tile_launch_args(nt, a, dA_array, ipiv_array, info_array, vb.count, stream);
         } else {
             SizeArgs sz{0, 0, 0, m_arr ? m_arr : n_arr, n_arr, ldda_arr, map};
-            rc = getrf_blocked_launch_sz(sz, vb.max_m, vb.max_n, dA_array, ipiv_array, info_array, vb.count, stream,
-                                         variant_nb(vb.variant));
-            if (rc == MAGMA_SUCCESS && solve && vb.max_nrhs > 0) {
+            // up to 16 right-hand sides go through the one-workgroup kernel with the matrix
+            const bool fused = vb.variant == kVbWg && solve && vb.max_nrhs <= 16;
+            if (vb.variant == kVbWg) {
+                WgRhs<double> rhs;
+                if (fused) {
+                    rhs.dB_array = dB_array;
+                    rhs.max_nrhs = vb.max_nrhs;
+                    rhs.nrhs_arr = nrhs_arr;
+                    rhs.lddb_arr = lddb_arr;
+                }
+                rc = getrf_wg_launch(sz, vb.max_m, dA_array, ipiv_array, info_array, rhs, vb.count, stream);
+            } else {
+                rc = getrf_blocked_launch_sz(sz, vb.max_m, vb.max_n, dA_array, ipiv_array, info_array, vb.count, stream,
+                                             variant_nb(vb.variant));
+            }
+            if (rc == MAGMA_SUCCESS && solve && !fused && vb.max_nrhs > 0) {
                 RsSizes rs{0, 0, 0, 0, vb.max_n, n_arr, nrhs_arr, ldda_arr, lddb_arr, map};
                 rc = getrs_generic_launch_t<double>(0, rs, vb.max_nrhs, dA_array, ipiv_array, dB_array, vb.count,
                                                     stream);
@@ -262,6 +282,8 @@ magma_int_t magma_dgetrf_vbatched_max_nocheck_work(magma_int_t* m, magma_int_t* 
     if (queue == nullptr) return MAGMA_ERR_NOT_INITIALIZED;
     hipSetDevice(queue->device);
     SizeArgs sz{0, 0, 0, m, n, ldda, nullptr};
+    if (getrf_wg_preferred(max_m, max_n, batchCount))
+        return getrf_wg_launch(sz, max_m, dA_array, dipiv_array, info_array, WgRhs<double>{}, batchCount, queue->stream);
     return getrf_blocked_launch_sz(sz, max_m, max_n, dA_array, dipiv_array, info_array, batchCount, queue->stream);
 }
 
