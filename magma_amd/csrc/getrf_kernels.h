@@ -71,6 +71,10 @@ size_t getrs_generic_bytes(int n, int elem);
 template <typename T>
 magma_int_t getrs_generic_launch_t(int trans, const RsSizes& sz, int max_nrhs, T** dA_array, int** ipiv_array,
                                    T** dB_array, int batch, hipStream_t stream);
+// getrs_wg.hip: one workgroup per system and 32 right-hand sides.
+template <typename T>
+magma_int_t getrs_wg_launch(int trans, const RsSizes& sz, int max_nrhs, T** dA_array, int** ipiv_array, T** dB_array,
+                            int batch, hipStream_t stream);
 size_t getrs_generic_bytes(int n);
 magma_int_t getrs_generic_launch(int trans, int n, int nrhs, double** dA_array, int ldda, int** ipiv_array,
                                  double** dB_array, int lddb, int batch, hipStream_t stream);

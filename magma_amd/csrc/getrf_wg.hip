@@ -38,6 +38,8 @@ namespace {
 typedef __bf16 wbf8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 wh8_t __attribute__((ext_vector_type(8)));
 
+constexpr int kWgGesvRhs = 16;      // right-hand sides carried along with the matrix
+
 template <typename T, int NTH>
 struct WgSmem {
     static constexpr int W = NTH / kWave;
@@ -52,7 +54,7 @@ struct WgSmem {
             T l11[NB * LD];                // the block's top 32 rows, l11[i*LD + j]
             int dst[NB];                   // where top row i went (below the block), or -1
         } f;
-        WgSweepSmem<T> sweep;
+        WgSweepSmem<T, kWgGesvRhs> sweep;
     };
     unsigned short map[NTH / NB][NTH];     // per block: position -> row before the block's interchanges
 };
@@ -525,7 +527,7 @@ template <typename T, int MODE>
 static magma_int_t wg_launch(const SizeArgs& sz, int max_m, T** dA_array, int** ipiv_array, int* info_array,
                              const WgRhs<T>& rhs, int batch, hipStream_t stream)
 {
-    if (!getrf_wg_supported(max_m) || rhs.max_nrhs > kWgMaxRhs) return MAGMA_ERR_NOT_SUPPORTED;
+    if (!getrf_wg_supported(max_m) || rhs.max_nrhs > kWgGesvRhs) return MAGMA_ERR_NOT_SUPPORTED;
     if (max_m <= 128)
         getrf_wg_kernel<T, MODE, 128><<<batch, 128, 0, stream>>>(sz, dA_array, ipiv_array, info_array, rhs);
     else if (max_m <= 256)

@@ -13,7 +13,6 @@
 namespace mgi {
 
 constexpr int kWgNB = 32;           // block width of the LU and of the sweeps
-constexpr int kWgMaxRhs = 32;       // right-hand sides one workgroup sweeps at once
 
 // v_mfma_*_16x16x4 layouts (lane l, lr = l % 16, lq = l / 16): first operand
 // P[lr][k = lq], second operand Q[k = lq][lr], result rows row(r, lq), column
@@ -167,52 +166,81 @@ __device__ __forceinline__ void wg_solve_block(const T* d, T (&y)[8], int q)
 
 // ---------------------------------------------------------------------------
 // Triangular sweep: B := E^{-1} B for one n x n triangle of the factors in A
-// (E = its transpose with TRANS), B column-major with nr <= kWgMaxRhs columns
-// in global memory, all waves of the workgroup. BACK runs from the last row
-// up. Per block of 32 rows: the diagonal block and the block's right-hand
-// sides go to LDS; one wave per 16 right-hand sides solves (lane 4c + q holds
-// rows q, q+4, ... of column c, the solved entry reaches the others of its
-// quad by DPP; reciprocal pivots); then every wave takes 16-row tiles of the
-// remaining rows and removes the block's contribution by MFMA, its operand
-// read straight from the factors. Each entry of the triangle is read once, so
-// the sweep is bound by HBM once enough workgroups hide the chain of blocks.
+// (E = its transpose with TRANS), B column-major with nr <= MAXR columns
+// in global memory or in LDS (PB), all waves of the workgroup. BACK runs from
+// the last row up. Per block of 32 rows: the diagonal block goes to LDS; one
+// wave per 16 right-hand sides solves it (wg_solve_block); then every wave takes
+// 16-row tiles of the remaining rows and removes the block's contribution by
+// MFMA, its operand read straight from the factors. The next diagonal block
+// and each wave's first tile are loaded while the block is solved. Each entry
+// of the triangle is read once, so the sweep is bound by HBM once enough
+// workgroups hide the chain of blocks.
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, int MAXR>
 struct WgSweepSmem {
     static constexpr int LD = kWgNB + 1;
     T d[kWgNB * LD];               // d[i*LD + j] = E(kb + i, kb + j)
-    T x[kWgMaxRhs * LD];           // x[c*LD + i]
+    T x[MAXR * LD];                // the block's right-hand sides, x[c*LD + i]
 };
 
-template <typename T, int NTH, bool BACK, bool TRANS, bool UNIT>
-__device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n, MGI_GLOBAL_AS T* B, int ldb, int nr,
-                                         WgSweepSmem<T>& sm)
+template <typename T, int NTH, bool BACK, bool TRANS, bool UNIT, typename PB, int MAXR>
+__device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n, PB B, int ldb, int nr,
+                                         WgSweepSmem<T, MAXR>& sm)
 {
-    constexpr int LD = WgSweepSmem<T>::LD;
+    constexpr int LD = WgSweepSmem<T, MAXR>::LD;
     constexpr int W = NTH / kWave;
+    constexpr int ND = kWgNB * kWgNB / NTH;        // diagonal-block entries per thread
     using M = WgMfma<T>;
     const int nblk = (n + kWgNB - 1) / kWgNB;
     const int nstr = (nr + 15) / 16;
+    auto block = [&](int ib) { return kWgNB * (BACK ? nblk - 1 - ib : ib); };
+    T dreg[ND];
+    // memory runs down i (or j when transposed); outside the block: identity
+    auto load_d = [&](int kb) {
+        const int nb = min(kWgNB, n - kb);
+#pragma unroll
+        for (int u = 0; u < ND; ++u) {
+            const int e = (int)threadIdx.x + NTH * u;
+            const int p = min(e % kWgNB, nb - 1), q = min(e / kWgNB, nb - 1);
+            dreg[u] = A[(kb + p) + (size_t)(kb + q) * ld];
+        }
+    };
+    load_d(block(0));
     for (int ib = 0; ib < nblk; ++ib) {
         const int t = threadIdx.x + wg_opaque_zero(), w = wg_wave(), l = t % kWave;
         const int lr = l % 16, lq = l / 16;
-        const int kb = kWgNB * (BACK ? nblk - 1 - ib : ib);
+        const int kb = block(ib);
         const int nb = min(kWgNB, n - kb);
-        // memory runs down i (or j when transposed); outside the block: identity
-        for (int e = t; e < kWgNB * kWgNB; e += NTH) {
-            const int p = e % kWgNB, q = e / kWgNB;
+#pragma unroll
+        for (int u = 0; u < ND; ++u) {
+            const int p = (t + NTH * u) % kWgNB, q = (t + NTH * u) / kWgNB;
             const int i = TRANS ? q : p, j = TRANS ? p : q;
             T v = i == j ? T(1) : T(0);
-            if (p < nb && q < nb && !(UNIT && i == j) && (BACK ? j >= i : j <= i)) v = A[(kb + p) + (size_t)(kb + q) * ld];
+            if (p < nb && q < nb && !(UNIT && i == j) && (BACK ? j >= i : j <= i)) v = dreg[u];
             sm.d[i * LD + j] = i == j ? T(1) / v : v;          // the diagonal as reciprocals
         }
         for (int e = t; e < kWgNB * 16 * nstr; e += NTH) {
             const int i = e % kWgNB, c = e / kWgNB;
             sm.x[c * LD + i] = (i < nb && c < nr) ? B[(kb + i) + (size_t)c * ldb] : T(0);
         }
+        if (ib + 1 < nblk) load_d(block(ib + 1));
+        // the rows not yet solved: below the block (a block with rows below
+        // is full), or above it
+        const int r0 = BACK ? 0 : kb + kWgNB, r1 = BACK ? kb : n;
+        const int tiles = r1 > r0 ? (r1 - r0 + 15) / 16 : 0;
+        auto load_e = [&](int ti, T (&ef)[8]) {
+            const int row = min(r0 + 16 * ti + lr, r1 - 1);
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) {
+                const int kc = kb + min(wg_k<T>(kk, lq), nb - 1);
+                ef[kk] = TRANS ? A[kc + (size_t)row * ld] : A[row + (size_t)kc * ld];
+            }
+        };
+        T ef[8];
+        if (w < tiles) load_e(w, ef);
         __syncthreads();
-        if (w < nstr) {
-            const int c = 16 * w + (l >> 2), q = l & 3;
+        for (int sw = w; sw < nstr; sw += W) {
+            const int c = 16 * sw + (l >> 2), q = l & 3;
             T y[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s) y[s] = sm.x[c * LD + q + 4 * s];
@@ -225,28 +253,18 @@ __device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n
             }
         }
         __syncthreads();
-        // the rows not yet solved: below the block (a block with rows below
-        // is full), or above it
-        const int r0 = BACK ? 0 : kb + kWgNB, r1 = BACK ? kb : n;
-        const int tiles = r1 > r0 ? (r1 - r0 + 15) / 16 : 0;
         for (int ti = w; ti < tiles; ti += W) {
             const int row = r0 + 16 * ti + lr;
             const bool rin = row < r1;
-            T ef[8];
+            T en[8];
+            if (ti + W < tiles) load_e(ti + W, en);
 #pragma unroll
-            for (int kk = 0; kk < 8; ++kk) {
-                const int k = wg_k<T>(kk, lq);
-                const int rc = min(row, r1 - 1), kc = kb + min(k, nb - 1);
-                const T e = TRANS ? A[kc + (size_t)rc * ld] : A[rc + (size_t)kc * ld];
-                ef[kk] = k < nb ? e : T(0);
-            }
+            for (int kk = 0; kk < 8; ++kk) ef[kk] = wg_k<T>(kk, lq) < nb ? ef[kk] : T(0);
             for (int s = 0; s < nstr; ++s) {
                 T bv[4];
 #pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int c = 16 * s + M::row(r, lq);
-                    bv[r] = B[min(row, r1 - 1) + (size_t)min(c, nr - 1) * ldb];
-                }
+                for (int r = 0; r < 4; ++r)
+                    bv[r] = B[min(row, r1 - 1) + (size_t)min(16 * s + M::row(r, lq), nr - 1) * ldb];
                 typename M::acc_t acc = {0, 0, 0, 0};
 #pragma unroll
                 for (int kk = 0; kk < 8; ++kk) acc = M::mma(sm.x[(16 * s + lr) * LD + wg_k<T>(kk, lq)], ef[kk], acc);
@@ -256,6 +274,8 @@ __device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n
                     if (rin && c < nr) B[row + (size_t)c * ldb] = bv[r] - acc[r];
                 }
             }
+#pragma unroll
+            for (int kk = 0; kk < 8; ++kk) ef[kk] = en[kk];
         }
         __syncthreads();
     }
