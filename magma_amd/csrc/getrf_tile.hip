@@ -41,6 +41,7 @@
 #include "magma_internal.h"
 #include "lu_device.h"
 #include "getrf_kernels.h"
+#include "wg_lu.h"
 
 #include <climits>
 
@@ -56,20 +57,6 @@ constexpr int kTileOwners = 3;      // waves 0..2 hold tiles, wave 3 factors pan
 // compiler uses global loads with a scalar base and a 32-bit lane offset
 // instead of 64-bit flat addresses.
 typedef MGI_GLOBAL_AS double gdouble;
-
-__device__ __forceinline__ double wave_max_d(double v)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = fmax(v, shfl_xor_d(v, off));
-    return v;
-}
-
-__device__ __forceinline__ int wave_min_i(int v)
-{
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v = min(v, __shfl_xor(v, off, kWave));
-    return v;
-}
 
 __device__ __forceinline__ int first_lane(unsigned long long mask) { return __ffsll((long long)mask) - 1; }
 
@@ -116,9 +103,12 @@ struct TileMap {
 // changes); only the ipiv and info writes are limited to real columns.
 //
 // The loop is software pipelined: step c updates column c+1 first, then
-// runs the pivot search of column c+1 (DPP maximum, ballots) in the same
-// branch-free block as the remaining rank-1 updates, so the reduction's
-// latency is hidden behind the FMAs.
+// runs the pivot search of column c+1 and the reciprocals of its candidates in
+// the same branch-free block as the remaining rank-1 updates, so the
+// reduction's and the division's latency is hidden behind the FMAs. The search
+// compares the upper 32 bits of |a| (which order like the values) by
+// DPP-sourced v_max_i32; only where they tie does a second search look at the
+// whole values.
 template <bool HAS1>
 __device__ __forceinline__ void panel_columns(double (&x0)[16], double (&x1)[16], int& pos0, int& pos1,
                                               bool& alive0, bool& alive1, int& info_local, MGI_GLOBAL_AS int* __restrict__ ipiv,
@@ -126,24 +116,36 @@ __device__ __forceinline__ void panel_columns(double (&x0)[16], double (&x1)[16]
 {
     // idamax candidates of column c: NaN never wins, except at the first
     // candidate position c, which keeps the pivot (counted as +inf)
-    double v0, v1 = -1.0, m;
+    double v0, v1 = -1.0, ri;
     unsigned long long b0, b1 = 0ull;
     auto search = [&](int c) {
-        v0 = alive0 ? fabs(x0[c]) : -1.0;
-        if (pos0 == c && v0 != v0) v0 = INFINITY;
+        v0 = fabs(x0[c]);
+        v0 = v0 == v0 ? v0 : (pos0 == c ? INFINITY : -1.0);
+        v0 = alive0 ? v0 : -1.0;
+        const int h0 = __double2hiint(v0);
+        int h = h0, h1 = 0;
         if (HAS1) {
-            v1 = alive1 ? fabs(x1[c]) : -1.0;
-            if (pos1 == c && v1 != v1) v1 = INFINITY;
+            v1 = fabs(x1[c]);
+            v1 = v1 == v1 ? v1 : (pos1 == c ? INFINITY : -1.0);
+            v1 = alive1 ? v1 : -1.0;
+            h1 = __double2hiint(v1);
+            h = max(h0, h1);
         }
-        m = wave_max_dpp(HAS1 ? fmax(v0, v1) : v0);
-        b0 = __ballot(v0 == m);
-        if (HAS1) b1 = __ballot(v1 == m);
+        // the reciprocal of the lane's larger candidate
+        ri = 1.0 / (HAS1 && h1 > h0 ? x1[c] : x0[c]);
+        const int mh = wg_group_max<64>(h);
+        b0 = __ballot(h0 == mh);
+        if (HAS1) b1 = __ballot(h1 == mh);
     };
+    int piv = 0;                                  // lane c: the position that step c's pivot came from
     search(0);
 #pragma unroll
     for (int c = 0; c < 16; ++c) {
-        if (__popcll(b0) + __popcll(b1) != 1) {
-            // exact tie: LAPACK keeps the lowest current position
+        const bool tie = __popcll(b0) + __popcll(b1) != 1;
+        if (tie) {
+            // equal upper halves: the largest value, then (an exact tie) LAPACK's
+            // lowest current position
+            const double m = wave_max_dpp(HAS1 ? fmax(v0, v1) : v0);
             const int cand = min(v0 == m ? pos0 : INT_MAX, (HAS1 && v1 == m) ? pos1 : INT_MAX);
             const int mpos = wave_min_dpp(cand);
             b0 = __ballot(v0 == m && pos0 == mpos);
@@ -156,7 +158,7 @@ __device__ __forceinline__ void panel_columns(double (&x0)[16], double (&x1)[16]
         const int cn = c + 1 < 16 ? c + 1 : c;      // next column (unused at c = 15)
         const double un = readlane_d(in1 ? x1[cn] : x0[cn], pl);
         const int pos_p = __builtin_amdgcn_readlane(in1 ? pos1 : pos0, pl);
-        if (l == 0 && k0 + c < n) ipiv[k0 + c] = k0 + pos_p + 1;
+        piv = l == c ? pos_p : piv;
         // LAPACK interchange of positions c and pos_p
         const bool me0 = !in1 && l == pl, me1 = in1 && l == pl;
         pos0 = me0 ? c : (pos0 == c ? pos_p : pos0);
@@ -166,9 +168,12 @@ __device__ __forceinline__ void panel_columns(double (&x0)[16], double (&x1)[16]
             alive1 = alive1 && !me1;
         }
         // multipliers: reciprocal scaling, or division when |pivot| < sfmin
-        const double rinv = 1.0 / pv;
+        // (a tie may leave the winner beside the reciprocal's candidate)
+        double rinv = readlane_d(ri, pl);
+        if (tie) rinv = 1.0 / pv;
         double l0 = x0[c] * rinv, l1 = HAS1 ? x1[c] * rinv : 0.0;
         if (!(pv != 0.0 && fabs(pv) >= kSfminD)) {
+            asm volatile("" ::: "memory");          // no division outside this branch
             if (pv != 0.0) {
                 l0 = x0[c] / pv;
                 if (HAS1) l1 = x1[c] / pv;
@@ -200,6 +205,7 @@ __device__ __forceinline__ void panel_columns(double (&x0)[16], double (&x1)[16]
             }
         }
     }
+    if (l < 16 && k0 + l < n) ipiv[k0 + l] = k0 + piv + 1;
 }
 
 // Barrier schedule shared by the two wave programs below (each __syncthreads
