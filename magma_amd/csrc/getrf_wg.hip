@@ -523,6 +523,13 @@ bool getrf_wg_preferred(int max_m, int max_n, int batch)
     return getrf_wg_supported(max_m) && (max_m < max_n ? max_m : max_n) > 12 && (max_n <= max_m || batch >= 512);
 }
 
+// The register-tile kernel has the shorter chain per system, but a CU holds
+// only two to four of them; from about six systems per CU on (1,536) the eight
+// that fit here win above 64 rows. Measured (gesv, FP64, us, tile against
+// this): 1,024 x 100^2 255 / 267, 2,048 x 100^2 478 / 371, 8,192 x 100^2 1781
+// / 1384, 20,000 x 128^2 5463 / 4560; at 64 rows 8,192 systems 508 / 588.
+bool getrf_wg_over_tile(int max_n, int batch) { return max_n > 64 && batch >= 1536; }
+
 template <typename T, int MODE>
 static magma_int_t wg_launch(const SizeArgs& sz, int max_m, T** dA_array, int** ipiv_array, int* info_array,
                              const WgRhs<T>& rhs, int batch, hipStream_t stream)

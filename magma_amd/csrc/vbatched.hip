@@ -6,7 +6,8 @@
 // src/zgetrf_vbatched.cpp:366-371). Here the sizes are grouped once into
 // n-buckets:
 //   * square n <= 128: the register-tile kernel instance for ceil(n/16)
-//     (fused with the solve when nrhs <= 16);
+//     (fused with the solve when nrhs <= 16), but many systems above 64 take
+//     the next;
 //   * up to 512 rows: the one-workgroup kernel, the solve included when nrhs
 //     <= 16;
 //   * larger or rectangular: the blocked path with a panel width per bucket,
@@ -109,7 +110,8 @@ static bool build_buckets(const int* h_m, const int* h_n, const int* h_nrhs, int
         if (v == kVbWg && !getrf_wg_supported(vb.max_m)) v = kVbAuto;
         if (variant_nb(v) != 0 && !blocked_nb_valid(vb.max_m, variant_nb(v))) v = kVbAuto;
         if (v == kVbAuto)
-            v = tile_ok ? kVbTile : getrf_wg_preferred(vb.max_m, vb.max_n, vb.count) ? kVbWg : kVbBlocked32;
+            v = tile_ok && !getrf_wg_over_tile(vb.max_n, vb.count) ? kVbTile
+                : getrf_wg_preferred(vb.max_m, vb.max_n, vb.count) ? kVbWg : kVbBlocked32;
         if (variant_nb(v) != 0 && !blocked_nb_valid(vb.max_m, variant_nb(v))) {
             v = blocked_nb_valid(vb.max_m, 16) ? kVbBlocked16 : kVbBlocked8;
         }

@@ -70,6 +70,17 @@ def test_gesv_edges(mb, oracle, n, nrhs, ld):
     assert np.array_equal(X[:, :, n:], B[:, :, n:])
 
 
+@pytest.mark.parametrize("n,nrhs", [(65, 1), (96, 16), (127, 3), (128, 4)])
+def test_gesv_many_small(mb, oracle, n, nrhs):
+    """1,536 systems of up to 128 rows: the line from the register-tile kernel."""
+    rng = np.random.default_rng(n)
+    A, B = uniform_batch(rng, 4, n), uniform_batch(rng, 4, n, cols=nrhs)
+    dA, dB = dev(np.tile(A, (384, 1, 1))), dev(np.tile(B, (384, 1, 1)))
+    ipiv, info = mb.dgesv_batched(dA, dB)
+    check(oracle, A, dA[-4:].cpu().numpy(), ipiv[-4:].cpu().numpy(), info[-4:].cpu().numpy(), n, n)
+    assert (oracle.gesv_backward_error(A, dB[-4:].cpu().numpy(), B, n) < TESTER_TOL).all()
+
+
 @pytest.mark.parametrize("n", [33, 64, 100, 129, 200, 300])
 def test_getrf_f32(mb, oracle, n):
     A = uniform_batch(np.random.default_rng(n), 3, n).astype(np.float32)
