@@ -32,6 +32,7 @@
 #include "magma_internal.h"
 #include "lu_device.h"
 #include "dense_kernels.h"
+#include "wg_lu.h"
 
 #include <cstdlib>
 #include <vector>
@@ -55,9 +56,6 @@ template <typename T> struct DLim;
 template <> struct DLim<double> { static constexpr double sfmin = kSfminD; };
 template <> struct DLim<float>  { static constexpr float sfmin = kSfminF; };
 
-__device__ __forceinline__ void argmax_t(double& v, int& idx) { wave_argmax(v, idx); }
-__device__ __forceinline__ void argmax_t(float& v, int& idx) { wave_argmax_f(v, idx); }
-
 // A wait gives up after this many ticks of the 100 MHz constant clock (2 s)
 // and raises the error word instead of spinning on.
 constexpr long long kDenseWaitTicks = 200000000LL;
@@ -71,6 +69,7 @@ typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
+typedef int int4v __attribute__((ext_vector_type(4)));
 
 }  // namespace
 
@@ -162,11 +161,17 @@ dense_panel_kernel(int m, int k, int jb, T* __restrict__ A, int lda, int* __rest
                 if (x != x) x = (pos == diag) ? T(INFINITY) : T(-1);
                 if (x >= T(0)) { v = x; vp = pos; }
             }
-            argmax_t(v, vp);
-            if (ln == 0) { s_wv[par][wv] = v; s_wp[par][wv] = vp; }
-            if (vp != INT_MAX && active && pos == vp) {
+            if (__ballot(vp != INT_MAX) != 0ull) {
+                const int pl = wg_pick<64>(v, vp);
+                if (ln == pl) {
+                    s_wv[par][wv] = v;
+                    s_wp[par][wv] = vp;
 #pragma unroll
-                for (int c = j; c < PW; ++c) s_cand[par][wv][c] = a[c];
+                    for (int c = j; c < PW; ++c) s_cand[par][wv][c] = a[c];
+                }
+            } else if (ln == 0) {
+                s_wv[par][wv] = T(-1);
+                s_wp[par][wv] = INT_MAX;
             }
             __syncthreads();
             // 2. wave 0: publish the workgroup's best, gather every
@@ -221,26 +226,37 @@ dense_panel_kernel(int m, int k, int jb, T* __restrict__ A, int lda, int* __rest
                     }
                     __builtin_amdgcn_s_sleep(1);
                 }
-                const int mycp = cp;
-                argmax_t(cv, cp);
-                const unsigned long long hit = __ballot(mycp == cp && cp != INT_MAX);
-                int gw = 0;
-                if (hit != 0ull) gw = __shfl(cg, __ffsll((long long)hit) - 1, kWave);
+                const unsigned long long hit = __ballot(cp != INT_MAX);
+                int gw = 0, pp = diag;
+                if (hit != 0ull) {
+                    const int pl = wg_pick<64>(cv, cp);
+                    gw = __builtin_amdgcn_readlane(cg, pl);
+                    pp = __builtin_amdgcn_readlane(cp, pl);
+                }
                 // only a timed-out wait can leave no candidate; keep the
                 // position in range then
-                int pp = cp;
                 if (pp < diag || pp >= m) pp = diag;
                 // the winning row, from the current column on
                 const unsigned long long* wsl = words + ((size_t)par * gmax + gw) * SW;
                 const unsigned long long t1 = __builtin_amdgcn_s_memrealtime();
                 for (;;) {
                     bool ok = true;
-                    for (int c = j + ln; c < PW; c += kWave) {
-                        const unsigned long long w0 = ld_word(wsl + 1 + c * NW);
-                        const unsigned long long w1 = NW == 2 ? ld_word(wsl + 1 + c * NW + 1) : w0;
-                        const bool good = hit != 0ull && (unsigned)(w0 >> 32) == tag && (unsigned)(w1 >> 32) == tag;
+                    // all of the row's words in one round trip
+                    constexpr int NC = (PW - j + kWave - 1) / kWave;
+                    unsigned long long w0[NC], w1[NC];
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        const int c = min(j + ln + kWave * q, PW - 1);
+                        w0[q] = ld_word(wsl + 1 + c * NW);
+                        w1[q] = NW == 2 ? ld_word(wsl + 1 + c * NW + 1) : w0[q];
+                    }
+#pragma unroll
+                    for (int q = 0; q < NC; ++q) {
+                        const int c = j + ln + kWave * q;
+                        if (c >= PW) continue;
+                        const bool good = hit != 0ull && (unsigned)(w0[q] >> 32) == tag && (unsigned)(w1[q] >> 32) == tag;
                         ok = ok && (good || hit == 0ull);
-                        s_u[par][c] = good ? value_of<T>((unsigned)w0, (unsigned)w1) : T(0);
+                        s_u[par][c] = good ? value_of<T>((unsigned)w0[q], (unsigned)w1[q]) : T(0);
                     }
                     if (__ballot(!ok) == 0ull) break;
                     if (ld_agent(w.err) != 0) break;
@@ -285,50 +301,54 @@ dense_panel_kernel(int m, int k, int jb, T* __restrict__ A, int lda, int* __rest
 // ---------------------------------------------------------------------------
 // Row pairs of the interchanges ipiv[s .. s+cnt) (LAPACK, 1-based, applied in
 // order): destination d receives the row found by tracing d back through
-// the interchanges. Destinations are the rows s .. s+cnt-1 and every
-// interchange partner below them (counted once). cnt <= kDenseMaxNB, one
-// thread per candidate destination (2 * kDenseMaxNB threads).
+// the interchanges. Candidate t < cnt is the row s + t, candidate cnt + i the
+// partner of step i where that lies below the block (at its first step only);
+// a candidate that nothing moves to has destination -1. cnt <= kDenseMaxNB,
+// one thread per candidate, 128 to a workgroup: both loops run over the whole
+// block, four steps per LDS read and without an early exit, so they are bound
+// by issue and spread over the CUs (one workgroup of 1,024 threads with a
+// read per step took 20 us of every block of 256, this 6).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(2 * kDenseMaxNB)
+constexpr int kPivmapThreads = 128;
+
+__global__ void __launch_bounds__(kPivmapThreads)
 dense_pivmap_kernel(const int* __restrict__ ipiv, int s, int cnt, int* __restrict__ pairs, int* __restrict__ npairs,
                     int maxp)
 {
-    __shared__ int piv[kDenseMaxNB];
-    __shared__ int count;
-    const int t = threadIdx.x;
-    if (t == 0) count = 0;
-    for (int i = t; i < cnt; i += blockDim.x) piv[i] = ipiv[s + i] - 1;
+    __shared__ __align__(16) int piv[kDenseMaxNB];
+    const int t = blockIdx.x * kPivmapThreads + threadIdx.x;
+    for (int i = threadIdx.x; i < kDenseMaxNB; i += kPivmapThreads) piv[i] = i < cnt ? ipiv[s + i] - 1 : -1;
     __syncthreads();
+    if (t == 0) *npairs = min(2 * cnt, maxp);
+    if (t >= 2 * cnt || t >= maxp) return;
     int d = -1;
     if (t < cnt) {
         d = s + t;
-    } else if (t < 2 * cnt) {
+    } else {
         const int i = t - cnt;
         const int p = piv[i];
-        if (p >= s + cnt) {
-            bool first = true;
-            for (int q = 0; q < i; ++q)
-                if (piv[q] == p) { first = false; break; }
-            if (first) d = p;
+        bool first = p >= s + cnt;
+#pragma unroll 4
+        for (int q = 0; q < cnt; q += 4) {
+            const int4v x = *reinterpret_cast<const int4v*>(&piv[q]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) first = first & !(q + u < i && x[u] == p);
+        }
+        if (first) d = p;
+    }
+    int row = d;
+#pragma unroll 4
+    for (int q = (cnt - 1) / 4 * 4; q >= 0; q -= 4) {
+        const int4v x = *reinterpret_cast<const int4v*>(&piv[q]);
+#pragma unroll
+        for (int u = 3; u >= 0; --u) {
+            const int k = s + q + u;
+            const int to = row == k ? x[u] : (row == x[u] ? k : row);
+            row = q + u < cnt ? to : row;
         }
     }
-    if (d >= 0) {
-        int row = d;
-        for (int i = cnt - 1; i >= 0; --i) {
-            const int p = piv[i];
-            if (row == s + i) row = p;
-            else if (row == p) row = s + i;
-        }
-        if (row != d) {
-            const int idx = atomicAdd(&count, 1);
-            if (idx < maxp) {
-                pairs[idx] = row;
-                pairs[maxp + idx] = d;
-            }
-        }
-    }
-    __syncthreads();
-    if (t == 0) *npairs = min(count, maxp);
+    pairs[t] = row;
+    pairs[maxp + t] = (d >= 0 && row != d) ? d : -1;
 }
 
 // Row moves of one block in the columns [c0, c1) and [c2, c3): one wave per
@@ -371,8 +391,11 @@ dense_laswp_kernel(int m, T* __restrict__ A, int lda, const int* __restrict__ pa
 // X + b*bs*bs (column-major, ld bs). UPPER = false: unit lower triangle;
 // UPPER = true: upper triangle with its diagonal. One wave per column of the
 // inverse (forward or back substitution on a unit vector); the triangle the
-// workgroup needs is staged in LDS, packed by columns. bs <= 256.
+// workgroup needs is staged in LDS, packed by columns. bs <= 128: lane l holds
+// rows l and l + 64 of its column.
 // ---------------------------------------------------------------------------
+constexpr int kTriSlots = 2;
+
 __host__ __device__ inline size_t trtri_lds_elems(int bs) { return (size_t)bs * (bs + 1) / 2; }
 
 template <typename T, bool UPPER>
@@ -391,50 +414,73 @@ dense_trtri_kernel(int n, int k0, int bs, const T* __restrict__ A, int lda, T* _
     // lower: columns p >= j0, rows p .. nb-1, column p at offset
     //   sum_{q=j0}^{p-1} (nb - q);  upper: columns p < min(nb, j0+4), rows 0..p at p(p+1)/2
     auto loff = [&](int p) -> int { return (p - j0) * nb - (p * (p - 1) / 2 - j0 * (j0 - 1) / 2); };
-    if (!UPPER) {
-        for (int p = j0 + wv; p < nb; p += 4) {
-            T* dstc = S + loff(p) - p;
-            for (int rr = p + ln; rr < nb; rr += kWave) dstc[rr] = D[rr + (size_t)p * lda];
+    // each wave's columns eight at a time: their loads are in flight together
+    // (one column at a time, the staging was most of this kernel's 34 us)
+    const int ns = (nb + kWave - 1) / kWave;
+    auto stage = [&](auto put, int pa, int pb) {
+        for (int p = pa + wv; p < pb; p += 32) {
+            T v[8][kTriSlots];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+#pragma unroll
+                for (int q = 0; q < kTriSlots; ++q)
+                    if (q < ns)
+                        v[u][q] = D[min(ln + kWave * q, nb - 1) + (size_t)min(p + 4 * u, pb - 1) * lda];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (p + 4 * u < pb) put(p + 4 * u, v[u]);
         }
+    };
+    if (!UPPER) {
+        stage([&](int p, T (&v)[kTriSlots]) {
+            T* dstc = S + loff(p) - p;
+#pragma unroll
+            for (int q = 0; q < kTriSlots; ++q) {
+                const int rr = ln + kWave * q;
+                if (rr >= p && rr < nb) dstc[rr] = v[q];
+            }
+        }, j0, nb);
     } else {
         const int pe = min(nb, j0 + 4);
-        for (int p = wv; p < pe; p += 4) {
+        stage([&](int p, T (&v)[kTriSlots]) {
             T* dstc = S + p * (p + 1) / 2;
-            for (int rr = ln; rr <= p; rr += kWave) dstc[rr] = D[rr + (size_t)p * lda];
-        }
+#pragma unroll
+            for (int q = 0; q < kTriSlots; ++q) {
+                const int rr = ln + kWave * q;
+                if (rr <= p) dstc[rr] = v[q];
+            }
+        }, 0, pe);
     }
     __syncthreads();
     const int j = j0 + wv;
     if (j >= nb) return;
-    T x[4];
+    T x[kTriSlots];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) x[s] = (ln + kWave * s == j) ? T(1) : T(0);
+    for (int s = 0; s < kTriSlots; ++s) x[s] = (ln + kWave * s == j) ? T(1) : T(0);
     if (!UPPER) {
-        for (int p = j; p < nb - 1; ++p) {
-            const int sp = p >> 6;
-            T xs = x[0];
-            if (sp == 1) xs = x[1];
-            else if (sp == 2) xs = x[2];
-            else if (sp == 3) xs = x[3];
-            const T xp = readlane_t(xs, p & 63);
-            const T* col = S + loff(p) - p;
+        // the entry of step p sits in slot p / 64; loads run ahead of the chain
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int rr = ln + kWave * s;
-                if (rr > p && rr < nb) x[s] = fma(-col[rr], xp, x[s]);
+        for (int sp = 0; sp < kTriSlots; ++sp) {
+            const int pe = min(nb - 1, 64 * (sp + 1));
+#pragma unroll 4
+            for (int p = max(j, 64 * sp); p < pe; ++p) {
+                const T* col = S + loff(p) - p;
+                const T xp = readlane_t(x[sp], p & 63);
+#pragma unroll
+                for (int s = sp; s < kTriSlots; ++s) {
+                    const int rr = ln + kWave * s;
+                    const T y = fma(-col[max(min(rr, nb - 1), p)], xp, x[s]);
+                    x[s] = (rr > p && rr < nb) ? y : x[s];
+                }
             }
         }
     } else {
         for (int p = j; p >= 0; --p) {
-            const int sp = p >> 6;
-            T xs = x[0];
-            if (sp == 1) xs = x[1];
-            else if (sp == 2) xs = x[2];
-            else if (sp == 3) xs = x[3];
+            const T xs = p >= kWave ? x[1] : x[0];
             const T* col = S + p * (p + 1) / 2;
             const T xp = readlane_t(xs, p & 63) / col[p];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < kTriSlots; ++s) {
                 const int rr = ln + kWave * s;
                 if (rr == p) x[s] = xp;
                 else if (rr < p) x[s] = fma(-col[rr], xp, x[s]);
@@ -443,7 +489,7 @@ dense_trtri_kernel(int n, int k0, int bs, const T* __restrict__ A, int lda, T* _
     }
     T* Xo = X + (size_t)b * bs * bs + (size_t)j * bs;
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
+    for (int s = 0; s < kTriSlots; ++s) {
         const int rr = ln + kWave * s;
         if (rr < nb) Xo[rr] = x[s];
     }
@@ -982,6 +1028,7 @@ void dense_work_carve(void* base, int m, int n, int elem, int gmax, DenseWork& w
 template <typename T>
 magma_int_t dense_trtri_launch(bool upper, int n, int k0, int bs, int nblk, const T* A, int lda, T* X, hipStream_t st)
 {
+    if (bs > kTriSlots * kWave) return MAGMA_ERR_NOT_SUPPORTED;
     const size_t lds = sizeof(T) * trtri_lds_elems(bs);
     dim3 grid((unsigned)ceildiv(bs, 4), (unsigned)nblk);
     if (upper) {
@@ -1082,7 +1129,7 @@ magma_int_t swaps_launch(int m, const int* ipiv, int s, int cnt, T* A, int lda, 
     const int ncol = (c1 - c0) + (c3 - c2);
     if (ncol <= 0 || cnt <= 0) return MAGMA_SUCCESS;
     if (cnt > kDenseMaxNB) return MAGMA_ERR_NOT_SUPPORTED;
-    dense_pivmap_kernel<<<1, 2 * kDenseMaxNB, 0, st>>>(ipiv, s, cnt, w.pairs, w.npairs, MP);
+    dense_pivmap_kernel<<<(unsigned)ceildiv(2 * cnt, kPivmapThreads), kPivmapThreads, 0, st>>>(ipiv, s, cnt, w.pairs, w.npairs, MP);
     MGI_LAUNCH_CHECK();
     // at most 2 cnt pairs: the row-move kernel holds that many per wave
     if (cnt <= 128)
