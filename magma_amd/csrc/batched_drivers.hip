@@ -178,6 +178,12 @@ namespace mgi {
 magma_int_t sgetrf_batched_async(int m, int n, float** dA_array, int ldda, int** ipiv_array, int* info_array,
                                  int batch, hipStream_t stream)
 {
+    // FP32 has no register-tile kernel: the wave kernel takes every batch (one
+    // system of 64 rows 160 -> 90 us, 20,000 x 8^2 156 -> 71, 8,192 x 64^2 787 -> 228)
+    if (m == n && n <= 64) {
+        TileArgs a{n, 0, ldda, 0, nullptr, nullptr, nullptr, nullptr, nullptr};
+        return slu_wave_launch((n + 15) / 16, a, dA_array, ipiv_array, info_array, batch, stream);
+    }
     if (getrf_wg_preferred(m, n, batch)) {
         SizeArgs sz{m, n, ldda, nullptr, nullptr, nullptr, nullptr};
         return sgetrf_wg_launch(kUpdF32, sz, m, dA_array, ipiv_array, info_array, WgRhs<float>{}, batch, stream);

@@ -123,6 +123,15 @@ struct TileArgs {
     const int* lddb_arr;
 };
 
+// getrf_wave.hip: square systems, one wave each; nch = ceil(max n / 16), at
+// most kLuWaveMaxD in FP64 and 4 in FP32. The FP64 form solves right-hand
+// sides too (dB_array not null).
+constexpr int kLuWaveMaxD = 3;
+magma_int_t lu_wave_launch(int nch, const TileArgs& a, double** dA_array, int** ipiv_array, int* info_array,
+                           double** dB_array, int batch, hipStream_t stream);
+magma_int_t slu_wave_launch(int nch, const TileArgs& a, float** dA_array, int** ipiv_array, int* info_array, int batch,
+                            hipStream_t stream);
+
 // getrf_tile.hip: square n <= 128, register-tiled, MFMA FP64 trailing update.
 // The *_args forms take per-matrix sizes; nt = ceil(max n / 16) selects the
 // kernel instance.

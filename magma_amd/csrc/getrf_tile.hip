@@ -704,6 +704,14 @@ template <bool WITH_B>
 static magma_int_t launch_nt(int nt, const TileArgs& a, double** dA_array, int** ipiv_array, int* info_array,
                              double** dB_array, int batch, hipStream_t stream)
 {
+    // one wave per system (getrf_wave.hip) carries more systems per CU at a
+    // longer chain each, and solves four right-hand sides at a time: from
+    // eight systems per CU on, up to 48 rows, with at most four of them
+    // (FP64 us, tile against wave: getrf 20,000 x 16^2 203 / 108, 2,048 x 48^2
+    // 108 / 103; gesv 4,096 x 32^2 r4 129 / 97, 8,192 x 32^2 r8 233 / 211,
+    // 20,000 x 32^2 r16 544 / 679; getrf 8,192 x 64^2 333 / 346)
+    if (nt <= kLuWaveMaxD && batch >= 2048 && (!WITH_B || (a.nrhs_arr == nullptr && a.nrhs <= 4)))
+        return lu_wave_launch(nt, a, dA_array, ipiv_array, info_array, dB_array, batch, stream);
     dim3 grid(batch), block(kTileThreads);
 #define MGI_TILE_CASE(NTV)                                                                               \
     case NTV:                                                                                            \

@@ -135,3 +135,49 @@ def test_same_as_blocked(mb, oracle, kind):
         f = np.isfinite(X)
         if kind == "zero_column":
             assert np.abs(X[f] - Y[f]).max() <= LU_FWD_TOL * np.abs(Y[f]).max()
+
+
+@pytest.mark.parametrize("n,nrhs,ld", [(1, 1, 1), (15, 4, 15), (16, 1, 20), (17, 3, 17), (32, 4, 32), (33, 2, 33),
+                                       (47, 4, 50), (48, 1, 48)])
+def test_wave_lu(mb, oracle, n, nrhs, ld):
+    """2,048 systems of up to 48 rows: one wave per system, FP64 LU and LU + solve."""
+    rng = np.random.default_rng(n * 7)
+    A, B = uniform_batch(rng, 8, n, ld=ld), uniform_batch(rng, 8, n, ld=ld, cols=nrhs)
+    A[1, :, :n] = rng.integers(-1, 2, (n, n))                # exact ties
+    A[2, n // 2, :n] = 0.0                                   # a zero column
+    A[1] += 3.0 * np.eye(n, ld)
+    tA, tB = np.tile(A, (256, 1, 1)), np.tile(B, (256, 1, 1))
+    dA, dB, dF = dev(tA), dev(tB), dev(tA)
+    ipiv, info = mb.dgesv_batched(dA, dB)
+    ipf, inf = mb.dgetrf_batched(dF, m=n)
+    assert torch.equal(dA, dF) and torch.equal(ipiv, ipf) and torch.equal(info, inf)
+    keep = [0, 1, 3, 4, 5, 6, 7]
+    last = np.array(keep) + 2040
+    LU, X = dA.cpu().numpy()[last], dB.cpu().numpy()[last]
+    check(oracle, A[keep], LU, ipiv.cpu().numpy()[last], info.cpu().numpy()[last], n, n)
+    assert int(info[2042]) == int(oracle.dgetrf(A[2:3], m=n)[2][0]) != 0
+    ok = info.cpu().numpy()[last] == 0
+    assert (oracle.gesv_backward_error(A[keep], X, B[keep], n)[ok] < TESTER_TOL).all()
+    assert np.array_equal(LU[:, :, n:], A[keep][:, :, n:]) and np.array_equal(X[:, :, n:], B[keep][:, :, n:])
+
+
+@pytest.mark.parametrize("n", [1, 5, 16, 31, 48, 49, 63, 64])
+def test_wave_lu_f32(mb, oracle, n):
+    """FP32 up to 64 rows against the FP64 oracle on small-integer systems
+    whose factors are exact, and by residual."""
+    rng = np.random.default_rng(n)
+    A = uniform_batch(rng, 5, n).astype(np.float32)
+    dA = dev(A)
+    ipiv, info = mb.sgetrf_batched(dA)
+    assert (info.cpu().numpy() == 0).all()
+    res = oracle.lu_residual(A.astype(np.float64), dA.cpu().numpy().astype(np.float64), ipiv.cpu().numpy(), n, n)
+    assert (res < 30 * np.finfo(np.float32).eps).all()
+    U = np.triu(rng.integers(-4, 5, (n, n))).astype(np.float32)
+    U[np.arange(n), np.arange(n)] = rng.integers(1, 10, n)
+    perm = rng.permutation(n)
+    P = np.empty_like(U)
+    P[perm] = U                                              # one non-zero candidate per column
+    dP = dev(np.ascontiguousarray(P.T)[None])
+    ip, inf = mb.sgetrf_batched(dP)
+    assert np.array_equal(dP.cpu().numpy()[0].T, U) and int(inf[0]) == 0
+    assert np.array_equal(ip.cpu().numpy()[0], oracle.dgetrf(np.ascontiguousarray(P.T.astype(np.float64))[None])[1][0])
