@@ -404,49 +404,13 @@ getrf_wg_kernel(SizeArgs sz, T** __restrict__ dA_array, int** __restrict__ ipiv_
                         lf[rt].x[v] = P[min(row0 + 16 * rt + lr, mloc - 1) + (size_t)Op::k(v, lq) * ld];
                     lf[rt].finish();
                 }
-                int s = task / nch;
-                if (row0 + 32 <= mloc) {
-                    // whole tiles: no guards, so that the loads of the next
-                    // strip stay in flight over the stores of this one (a
-                    // guarded store makes the wait counts unknown)
-                    const size_t offu = (size_t)lr * ld + Op::k(0, lq);
-                    const size_t offc = (size_t)M::row(0, lq) * ld + row0 + lr;
-                    const size_t stepc = (size_t)(M::row(1, 0) - M::row(0, 0)) * ld;
-                    auto load_u = [&](int q, Op& u) {
-                        auto Uc = A + k + (size_t)(k + NB + 16 * q) * ld + offu;
-#pragma unroll
-                        for (int v = 0; v < 8; ++v) u.x[v] = Uc[Op::k(v, 0)];
-                    };
-                    auto tile = [&](int q, Op& u, Op& un) {
-                        auto Cc = A + k + (size_t)(k + NB + 16 * q) * ld + offc;
-                        T c[2][4];
-#pragma unroll
-                        for (int r = 0; r < 4; ++r)
-#pragma unroll
-                            for (int rt = 0; rt < 2; ++rt) c[rt][r] = Cc[r * stepc + 16 * rt];
-                        load_u(min(q + ncg, nfull - 1), un);
-                        u.finish();
-#pragma unroll
-                        for (int rt = 0; rt < 2; ++rt) {
-                            acc_t acc = {0, 0, 0, 0};
-                            acc = upd_mma<T, MODE>(u, lf[rt], acc);
-#pragma unroll
-                            for (int r = 0; r < 4; ++r) Cc[r * stepc + 16 * rt] = c[rt][r] - acc[r];
-                        }
-                    };
-                    if (s < nfull) {
-                        Op u0, u1;
-                        load_u(s, u0);
-                        for (; s < nfull; s += 2 * ncg) {
-                            tile(s, u0, u1);
-                            if (s + ncg < nfull) tile(s + ncg, u1, u0);
-                        }
-                        // first strip of this wave that is left
-                        s = task / nch;
-                        s += (nfull - s + ncg - 1) / ncg * ncg;
-                    }
-                }
-                for (; s < ns; s += ncg) {
+                // Strips from the right: those that the interchanges touched
+                // last come first, and the next panel's columns are written
+                // last, while the L2 still holds them
+                const int s0 = task / nch;
+                const bool whole = row0 + 32 <= mloc;
+                const int last = s0 < ns ? s0 + (ns - 1 - s0) / ncg * ncg : -1;    // this wave's last strip
+                for (int s = last; s >= (whole ? max(nfull, s0) : s0); s -= ncg) {
                     const Strip<T> x = strip(s);
                     Op u;
                     T c[2][4];
@@ -470,6 +434,43 @@ getrf_wg_kernel(SizeArgs sz, T** __restrict__ dA_array, int** __restrict__ ipiv_
                                 if (M::row(r, lq) < x.nc)
                                     x.p[row0 + 16 * rt + lr + (size_t)M::row(r, lq) * x.ld] = c[rt][r] - acc[r];
                         }
+                    }
+                }
+                if (whole && s0 < nfull) {
+                    // whole tiles: no guards, so that the loads of the next
+                    // strip stay in flight over the stores of this one (a
+                    // guarded store makes the wait counts unknown)
+                    const size_t offu = (size_t)lr * ld + Op::k(0, lq);
+                    const size_t offc = (size_t)M::row(0, lq) * ld + row0 + lr;
+                    const size_t stepc = (size_t)(M::row(1, 0) - M::row(0, 0)) * ld;
+                    auto load_u = [&](int q, Op& u) {
+                        auto Uc = A + k + (size_t)(k + NB + 16 * q) * ld + offu;
+#pragma unroll
+                        for (int v = 0; v < 8; ++v) u.x[v] = Uc[Op::k(v, 0)];
+                    };
+                    auto tile = [&](int q, Op& u, Op& un) {
+                        auto Cc = A + k + (size_t)(k + NB + 16 * q) * ld + offc;
+                        T c[2][4];
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+#pragma unroll
+                            for (int rt = 0; rt < 2; ++rt) c[rt][r] = Cc[r * stepc + 16 * rt];
+                        load_u(max(q - ncg, 0), un);
+                        u.finish();
+#pragma unroll
+                        for (int rt = 0; rt < 2; ++rt) {
+                            acc_t acc = {0, 0, 0, 0};
+                            acc = upd_mma<T, MODE>(u, lf[rt], acc);
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) Cc[r * stepc + 16 * rt] = c[rt][r] - acc[r];
+                        }
+                    };
+                    Op u0, u1;
+                    int s = s0 + (nfull - 1 - s0) / ncg * ncg;
+                    load_u(s, u0);
+                    for (; s >= 0; s -= 2 * ncg) {
+                        tile(s, u0, u1);
+                        if (s - ncg >= 0) tile(s - ncg, u1, u0);
                     }
                 }
             }
