@@ -576,6 +576,7 @@ def main():
     achieved = bytes_step / ev_avg_s / 1e9
     workload = f"dgesv_batched {batch} x {n}x{n} FP64, nrhs={nrhs}, ldda={n}"
     fused = n <= 128 and nrhs <= 16
+    wg = fused and n > 64 and batch >= 1536      # the same line as getrf_wg_over_tile
     roof = {
         "bound": "hbm",
         "achieved": round(achieved, 1),
@@ -583,7 +584,8 @@ def main():
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4),
         "traffic": measured_traffic(workload),
-        "kernel": (f"getrf_tile_kernel<{(n + 15) // 16}, true> (one fused LU + solve launch per call)" if fused
+        "kernel": ("getrf_wg_kernel<double, 128> (one fused LU + solve launch per call)" if wg else
+                   f"getrf_tile_kernel<{(n + 15) // 16}, true> (one fused LU + solve launch per call)" if fused
                    else "magma_dgesv_batched launch group (getrf + getrs)"),
         "event_ms_avg": round(ev_avg_s * 1e3, 4),
         "algorithmic_bytes_per_launch": bytes_step,

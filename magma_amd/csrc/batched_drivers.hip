@@ -137,10 +137,11 @@ magma_int_t magma_dgesv_batched(magma_int_t n, magma_int_t nrhs, double** dA_arr
 
 void magma_get_dgetrf_batched_nbparam(magma_int_t n, magma_int_t* nb, magma_int_t* recnb)
 {
-    // The blocking the square n x n batched LU uses: the register-tile kernel
-    // factors 16-column panels; the LDS kernel factors the whole matrix one
-    // column at a time; the blocked LU factors nb-wide blocks of 32-wide
-    // panels.
+    // The blocking a caller that sizes its own workspace may plan with: 16 for
+    // the register-tile orders, the whole matrix where it fits a workgroup's
+    // LDS, and above that the blocked LU's nb-wide blocks of 32-wide panels.
+    // The one-workgroup kernel takes some of these orders with 32-wide panels
+    // in place; it needs no workspace, so the answer does not depend on it.
     int b = 16, r = 16;
     if (!mgi::getrf_tile_supported(n)) {
         if (mgi::getrf_lds_bytes(n, n) <= mgi::max_dynamic_lds()) {
@@ -157,8 +158,9 @@ void magma_get_dgetrf_batched_nbparam(magma_int_t n, magma_int_t* nb, magma_int_
 
 void magma_get_dgetrf_vbatched_nbparam(magma_int_t max_m, magma_int_t max_n, magma_int_t* nb, magma_int_t* recnb)
 {
-    // The vbatched LU puts systems up to 128 on the register tile (16-column
-    // panels) and larger ones on the blocked LU sized by the largest row count.
+    // 16 (the register tile's panels) up to 128 rows, the blocked LU's block
+    // for the largest row count above that; see the square form above for the
+    // one-workgroup kernel.
     int b = 16, r = 16;
     if (max_m > 128 || max_n > 128) {
         b = std::max(mgi::getrf_blocked_nb(max_m), 1);

@@ -16,8 +16,8 @@ constexpr int kRsThreads = 256;
 // value reaches the other lanes through a cross-lane read, and the factor is
 // streamed down its columns (64 contiguous elements per slot, loads issued
 // ahead of the dependent updates). The interchanges are applied by tracing
-// every row back through them, as in the kernel above; the per-row operation
-// order is that of the column-oriented sweeps above.
+// every row back through them; each row's updates run in the order of the
+// columns, forward and then backward.
 // ---------------------------------------------------------------------------
 constexpr int kWaveCols = 4;
 
