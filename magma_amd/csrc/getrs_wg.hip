@@ -10,10 +10,14 @@
 //
 // Bound: HBM on the factors once a CU holds several workgroups; a single
 // system is bound by the chain of its 32-row blocks. Against the sweeps with
-// per-row FMA that it replaced (us): FP64 1,000 x 384^2 transposed, 16
-// right-hand sides 1219 -> 553 (2.1 TB/s on the factors); FP64 8,192 x 64^2
-// transposed, 8 right-hand sides 563 -> 167; FP32 1,000 x 300^2, 8 right-hand
-// sides 6849 -> 167.
+// per-row FMA that it replaced (kernel, us): FP64 1,000 x 384^2 transposed, 16
+// right-hand sides 1219 -> 601 (2.0 TB/s on the factors); FP64 8,192 x 64^2
+// transposed, 8 right-hand sides 562 -> 209; FP32 the same 372 -> 82; FP32
+// 1,000 x 300^2, 8 right-hand sides 6849 -> 157. At small orders the chain of
+// one wave counts: one division per diagonal block instead of one per entry
+// that a thread holds, and eight columns of B in flight instead of one, took
+// whole calls of 8,192 x 64^2 r8 from 265 to 230 us (FP32 111 to 95) and of
+// 20,000 x 16^2 r16 from 377 to 255.
 #include "magma_internal.h"
 #include "getrf_kernels.h"
 #include "wg_lu.h"
@@ -70,8 +74,19 @@ getrs_wg_kernel(RsSizes sz, T** __restrict__ dA_array, int** __restrict__ ipiv_a
     __syncthreads();
     if constexpr (INLDS) {
         const int ldx = n | 1;                 // odd: the columns start in different banks
-        for (int c = 0; c < nr; ++c)
-            for (int i = tid; i < n; i += NTH) buf[i + c * ldx] = B[(TRANS ? i : perm[i]) + (size_t)c * lddb];
+        // eight columns' loads in flight at a time (those past the last one
+        // read it again and are dropped)
+        for (int i = tid; i < n; i += NTH) {
+            auto Bi = B + (TRANS ? i : perm[i]);
+            for (int c = 0; c < nr; c += 8) {
+                T v[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = Bi[(size_t)min(c + e, nr - 1) * lddb];
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (c + e < nr) buf[i + (c + e) * ldx] = v[e];
+            }
+        }
         __syncthreads();
         if constexpr (TRANS) {
             wg_sweep<T, NTH, false, true, false>(A, ldda, n, buf, ldx, nr, sm);     // U^T

@@ -211,13 +211,21 @@ __device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n
         const int lr = l % 16, lq = l / 16;
         const int kb = block(ib);
         const int nb = min(kWgNB, n - kb);
+        T dg = T(1);
 #pragma unroll
         for (int u = 0; u < ND; ++u) {
             const int p = (t + NTH * u) % kWgNB, q = (t + NTH * u) / kWgNB;
             const int i = TRANS ? q : p, j = TRANS ? p : q;
             T v = i == j ? T(1) : T(0);
             if (p < nb && q < nb && !(UNIT && i == j) && (BACK ? j >= i : j <= i)) v = dreg[u];
-            sm.d[i * LD + j] = i == j ? T(1) / v : v;          // the diagonal as reciprocals
+            dg = i == j ? v : dg;
+            sm.d[i * LD + j] = v;
+        }
+        if constexpr (!UNIT) {
+            // the diagonal as reciprocals: each thread holds at most one of
+            // its entries, so one division serves the block
+            const int p = t % kWgNB;
+            if (p % (NTH / kWgNB) == t / kWgNB) sm.d[p * LD + p] = T(1) / dg;
         }
         for (int e = t; e < kWgNB * 16 * nstr; e += NTH) {
             const int i = e % kWgNB, c = e / kWgNB;
