@@ -20,6 +20,7 @@ constexpr int kRsThreads = 256;
 // columns, forward and then backward.
 // ---------------------------------------------------------------------------
 constexpr int kWaveCols = 4;
+constexpr int kFewSystems = 1024;     // FP64 batches that do not fill the chip with one wave per system
 
 template <typename T, int R>
 __global__ void __launch_bounds__(kRsThreads)
@@ -186,12 +187,19 @@ magma_int_t getrs_generic_launch_t(int trans, const RsSizes& sz, int max_nrhs, T
 {
     if (batch <= 0 || max_nrhs <= 0) return MAGMA_SUCCESS;
     if (getrs_generic_bytes(sz.max_n, sizeof(T)) > max_dynamic_lds()) return MAGMA_ERR_NOT_SUPPORTED;
-    // up to four right-hand sides of a system of up to 256 rows read the
+    // up to four right-hand sides of many systems of up to 256 rows read the
     // factors once in one wave, without barriers (FP64 us, wave against
-    // workgroup: 2,000 x 256^2 r1 274 / 307, 20,000 x 16^2 r2 85 / 145, 8,192
-    // x 64^2 r1 137 / 153); with more, or above 256 rows, the workgroup's MFMA
-    // sweeps win (2,000 x 256^2 r16 935 / 408, 5,000 x 100^2 r5 361 / 226)
-    if (trans == 0 && sz.max_n <= 256 && max_nrhs <= kWaveCols) {
+    // workgroup: 2,000 x 256^2 r1 276 / 379, r4 320 / 382; 20,000 x 16^2 r2 85 /
+    // 222; 8,192 x 64^2 r1 134 / 212; 5,000 x 100^2 r4 219 / 284); with more, or
+    // above 256 rows, the workgroup's MFMA sweeps win (2,000 x 256^2 r16 935 /
+    // 486, 5,000 x 100^2 r5 361 / 286). Up to four systems per CU the wave's
+    // chain of columns is what counts, and the workgroup's chain of blocks is
+    // shorter (64 x 256^2 r1 174 / 106, r4 221 / 106; 1,024 x 256^2 r1 231 / 199;
+    // 1,024 x 64^2 r4 56 / 38; even at 16 rows). FP32 batches, whose waves
+    // stream half the bytes, stay with the wave at every size (8,192 x 64^2 r1
+    // 80 / 89), and so do mapped buckets, beside which other buckets run.
+    const bool few = sizeof(T) == 8 && sz.map == nullptr && batch <= kFewSystems;
+    if (trans == 0 && sz.max_n <= 256 && max_nrhs <= kWaveCols && !few) {
         if (sz.max_n <= 64) return getrs_wave_launch<T, 1>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
         if (sz.max_n <= 128) return getrs_wave_launch<T, 2>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
         return getrs_wave_launch<T, 4>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);

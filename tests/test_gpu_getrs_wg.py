@@ -51,3 +51,23 @@ def test_getrs(oracle, trans, n, nrhs, pad):
         Xs, Bs = dBs[s].cpu().numpy().astype(np.float64).T, B[s].astype(np.float32).astype(np.float64).T
         r = np.abs(Bs - Pop @ Xs).max() / (n * np.abs(L).sum(1).max() * np.abs(U).sum(1).max() * np.abs(Xs).max())
         assert r < 30 * np.finfo(np.float32).eps, r
+
+
+@pytest.mark.parametrize("batch", [1024, 1025])
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (16, 4), (64, 1), (65, 3), (129, 4), (256, 2)])
+def test_getrs_few_and_many(oracle, batch, n, nrhs):
+    """Both sides of the line between one workgroup and one wave per system:
+    three systems repeated through the batch, every copy with the same answer."""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from magma_amd import batched as mb
+    rng = np.random.default_rng(n * 7 + nrhs)
+    A, B = uniform_batch(rng, 3, n, ld=n), uniform_batch(rng, 3, n, ld=n, cols=nrhs)
+    LU, piv, _ = oracle.dgetrf(A, m=n)
+    pick = torch.arange(batch) % 3
+    dB = torch.from_numpy(B)[pick].cuda()
+    mb.dgetrs_batched(111, torch.from_numpy(LU)[pick].cuda(), torch.from_numpy(piv)[pick].cuda(), dB)
+    X = dB.cpu()
+    assert torch.equal(X, X[:3][pick])
+    be = oracle.gesv_backward_error(A, X[:3].numpy(), B, n)
+    assert (be < TESTER_TOL).all(), be.max()
