@@ -122,4 +122,13 @@ def load_variants(n=None, nrhs=None, path: Path = CACHE, tune_missing: bool = Tr
                 mine[b] = v
             path.parent.mkdir(parents=True, exist_ok=True)
             path.write_text(json.dumps(table, indent=1, sort_keys=True) + "\n")
+    if n is not None:
+        # The cached choice was timed on a full bucket. With fewer systems than
+        # the line that uniform batches have (getrf_wg_over_tile), a bucket of
+        # 65..128 rows is bound by one system's chain, which is shorter on the
+        # tile (27 systems of 50..91 rows: 116 us a replay against 161).
+        ids = bucket_of(np.asarray(n))
+        for b, v in mine.items():
+            if v == 6 and 4 <= b <= 7 and np.count_nonzero(ids == b) < 1536:
+                mine[b] = 1
     return mine
