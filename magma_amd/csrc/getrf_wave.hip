@@ -108,22 +108,21 @@ lu_wave_kernel(TileArgs ta, T** __restrict__ dA_array, int** __restrict__ ipiv_a
                 rdiag = win ? rinv : rdiag;
                 const bool zero = __ballot(pv == T(0)) != 0ull;
                 if (zero && info == 0) info = k + 1;
-                if (!zero) {
-                    T f = a[j] * rinv;
-                    if (__ballot(fabs(pv) < WgLim<T>::sfmin) != 0ull) {
-                        asm volatile("" ::: "memory");     // no division outside this branch
-                        f = a[j] / pv;
-                    }
-                    if (active) {
-                        a[j] = f;
+                // a zero pivot leaves its column unscaled; the step is applied
+                // all the same (LAPACK dgetf2)
+                T f = a[j] * rinv;
+                if (__ballot(fabs(pv) < WgLim<T>::sfmin) != 0ull) {
+                    asm volatile("" ::: "memory");     // no division outside this branch
+                    f = zero ? a[j] : a[j] / pv;
+                }
+                if (active) {
+                    a[j] = f;
 #pragma unroll
-                        for (int c = j + 1; c < 16; ++c) a[c] = fma(-f, u[c], a[c]);
-                    }
+                    for (int c = j + 1; c < 16; ++c) a[c] = fma(-f, u[c], a[c]);
                 }
             }
         });
-        // the same steps on the later groups (a zero pivot's multipliers were
-        // left as they are: all zero)
+        // the same steps on the later groups
         const int steps = min(16, n - 16 * h);
         wg_for(std::make_integer_sequence<int, NCH - 1>{}, [&](auto gc) {
             constexpr int g = decltype(gc)::value + 1;

@@ -249,17 +249,17 @@ getrf_wg_kernel(SizeArgs sz, T** __restrict__ dA_array, int** __restrict__ ipiv_
                         pos = (active & first) ? p : pos;
                         pos = win ? j0 + j : pos;
                         active = active & !win;
-                        if (!zero) {
-                            T f = a[j] * rinv;
-                            if (__ballot(fabs(pv) < WgLim<T>::sfmin) != 0ull) {
-                                asm volatile("" ::: "memory");     // no division outside this branch
-                                f = a[j] / pv;
-                            }
-                            if (active) {
-                                a[j] = f;
+                        // a zero pivot leaves its column unscaled; the step
+                        // is applied all the same (LAPACK dgetf2)
+                        T f = a[j] * rinv;
+                        if (__ballot(fabs(pv) < WgLim<T>::sfmin) != 0ull) {
+                            asm volatile("" ::: "memory");     // no division outside this branch
+                            f = zero ? a[j] : a[j] / pv;
+                        }
+                        if (active) {
+                            a[j] = f;
 #pragma unroll
-                                for (int c = j + 1; c < 16; ++c) a[c] = fma(-f, u[c], a[c]);
-                            }
+                            for (int c = j + 1; c < 16; ++c) a[c] = fma(-f, u[c], a[c]);
                         }
                     }
                 });

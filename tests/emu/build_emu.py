@@ -131,9 +131,9 @@ def build(src: Path | None = None) -> Path:
     gen = BUILD / "src"
     objd = BUILD / "obj"
     objd.mkdir(parents=True, exist_ok=True)
-    cpps = transform(src, gen) + [HERE / "emu.cpp"]
+    cpps = transform(src, gen) + [HERE / "emu.cpp", HERE / "forms.cpp"]
     flags = ["-w", "-std=c++20", "-O1", "-g", "-fsanitize=address", "-fno-omit-frame-pointer", "-fPIC",
-             f"-I{HERE / 'include'}", f"-I{ROOT / 'include'}"]
+             f"-I{HERE / 'include'}", f"-I{ROOT / 'include'}", f"-I{gen}"]
 
     headers = [h for h in gen.glob("*.h")] + [HERE / "include" / "hip" / "hip_runtime.h"]
     newest_h = max(h.stat().st_mtime for h in headers)

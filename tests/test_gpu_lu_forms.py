@@ -1,0 +1,51 @@
+"""Inputs on which the batched LU kernels must follow LAPACK step by step, at
+batch sizes on both sides of the lines between the kernels, against the
+oracle."""
+import sys
+from pathlib import Path
+
+import numpy as np
+import pytest
+
+from conftest import EPS
+
+torch = pytest.importorskip("torch")
+
+sys.path.insert(0, str(Path(__file__).resolve().parent / "emu"))
+
+import lu_inputs  # noqa: E402
+
+pytestmark = pytest.mark.gpu
+
+LU_FWD_TOL = 1e3 * EPS
+
+
+@pytest.fixture(scope="module")
+def mb():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from magma_amd import batched
+    return batched
+
+
+@pytest.mark.parametrize("n,batch,cols", [(32, 2047, [0]), (32, 2048, [0]), (48, 2048, [3, 20]), (80, 1535, [0]),
+                                          (80, 1536, [0]), (130, 2, [5, 20, 40]), (300, 2, [0, 70])])
+def test_zero_pivot_above_a_nan(mb, oracle, n, batch, cols):
+    A = lu_inputs.zero_columns_with_nan(np.random.default_rng(n), n, cols)
+    dA = torch.from_numpy(A).cuda().repeat(batch, 1, 1)
+    ipiv, info = mb.dgetrf_batched(dA)
+    LUo, ipo, info_o = oracle.dgetrf(A)
+    assert (info.cpu().numpy() == info_o[0]).all()
+    assert (ipiv.cpu().numpy() == ipo[0]).all()
+    if batch >= 1536 or n > 128:          # the register tile spreads a NaN over its 16-row blocks
+        assert np.array_equal(np.isfinite(dA[-1].cpu().numpy()), np.isfinite(LUo[0]))
+
+
+@pytest.mark.parametrize("m,n,zeros", [(80, 80, [0]), (130, 130, [5, 20, 40]), (64, 20, [17])])
+def test_zero_pivot_without_pivoting(mb, oracle, m, n, zeros):
+    M = lu_inputs.dominant_with_zeros(np.random.default_rng(m), m, n, zeros)
+    ref, info_ref = lu_inputs.getf2_nopiv(M)
+    dA = torch.from_numpy(np.ascontiguousarray(M.T)[None]).cuda()
+    info = mb.dgetrf_nopiv_batched(dA, m=m)
+    assert int(info[0]) == info_ref
+    assert oracle.lu_forward_error(ref.T[None], dA.cpu().numpy(), m)[0] < LU_FWD_TOL
