@@ -664,8 +664,13 @@ __device__ __forceinline__ void panel_wave_main(const TileCtx<NT, WITH_B>& cx)
     }
 }
 
+// Waves per SIMD, that is workgroups per CU, to compile for. The LU alone of
+// 65..80 rows keeps three (at 172 registers, without the bound, two: 513..768
+// systems then take a second round, 700 x 80^2 130 us against 90).
+constexpr int tile_per_cu(int nt, bool with_b) { return !with_b && nt == 5 ? 3 : 2; }
+
 template <int NT, bool WITH_B>
-__global__ void __launch_bounds__(kTileThreads, 2)
+__global__ void __launch_bounds__(kTileThreads, tile_per_cu(NT, WITH_B))
 getrf_tile_kernel(TileArgs ta, double** __restrict__ dA_array, int** __restrict__ ipiv_array,
                   int* __restrict__ info_array, double** __restrict__ dB_array)
 {
