@@ -138,29 +138,35 @@ __device__ __forceinline__ float wg_quad(float v)
 // or upper triangular and solved from the last row up with BACK; with DIAG its
 // diagonal holds reciprocal pivots, without it is one. A row that a step does
 // not reach keeps its value whatever the step's factors are (a select, not a
-// zero factor: an infinite entry stays in its row).
+// zero factor: an infinite entry stays in its row). Rows from nb on are an
+// identity with a zero right-hand side; the groups of four steps that hold
+// only such rows are skipped.
 template <typename T, bool BACK, bool DIAG = false>
-__device__ __forceinline__ void wg_solve_block(const T* d, T (&y)[8], int q)
+__device__ __forceinline__ void wg_solve_block(const T* d, T (&y)[8], int q, int nb = kWgNB)
 {
     constexpr int LD = kWgNB + 1;
-    wg_for(std::make_integer_sequence<int, kWgNB>{}, [&](auto kc) {
-        constexpr int k = BACK ? kWgNB - 1 - decltype(kc)::value : decltype(kc)::value;
-        constexpr int sk = k >> 2, qk = k & 3;
+    wg_for(std::make_integer_sequence<int, kWgNB / 4>{}, [&](auto gc) {
+        constexpr int g = BACK ? kWgNB / 4 - 1 - decltype(gc)::value : decltype(gc)::value;
+        if (4 * g >= nb) return;
         // four steps' coefficients in flight at a time
-        if constexpr (decltype(kc)::value % 4 == 0) __builtin_amdgcn_sched_barrier(0);
-        if constexpr (DIAG) {
-            const T v = y[sk] * d[k * LD + k];
-            y[sk] = q == qk ? v : y[sk];
-        }
-        const T xk = wg_quad<qk>(y[sk]);
+        __builtin_amdgcn_sched_barrier(0);
+        wg_for(std::make_integer_sequence<int, 4>{}, [&](auto kc) {
+            constexpr int qk = BACK ? 3 - decltype(kc)::value : decltype(kc)::value;
+            constexpr int sk = g, k = 4 * g + qk;
+            if constexpr (DIAG) {
+                const T v = y[sk] * d[k * LD + k];
+                y[sk] = q == qk ? v : y[sk];
+            }
+            const T xk = wg_quad<qk>(y[sk]);
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            if (BACK ? 4 * s >= k : 4 * s + 3 <= k) continue;          // every row of the slot is done
-            const int i = q + 4 * s;
-            const T v = fma(-d[i * LD + k], xk, y[s]);
-            const bool whole = BACK ? 4 * s + 3 < k : 4 * s > k;       // every row of the slot is reached
-            y[s] = (whole || (BACK ? i < k : i > k)) ? v : y[s];
-        }
+            for (int s = 0; s < 8; ++s) {
+                if (BACK ? 4 * s >= k : 4 * s + 3 <= k) continue;          // every row of the slot is done
+                const int i = q + 4 * s;
+                const T v = fma(-d[i * LD + k], xk, y[s]);
+                const bool whole = BACK ? 4 * s + 3 < k : 4 * s > k;       // every row of the slot is reached
+                y[s] = (whole || (BACK ? i < k : i > k)) ? v : y[s];
+            }
+        });
     });
 }
 
@@ -252,7 +258,7 @@ __device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n
             T y[8];
 #pragma unroll
             for (int s = 0; s < 8; ++s) y[s] = sm.x[c * LD + q + 4 * s];
-            wg_solve_block<T, BACK, !UNIT>(sm.d, y, q);
+            wg_solve_block<T, BACK, !UNIT>(sm.d, y, q, nb);
 #pragma unroll
             for (int s = 0; s < 8; ++s) {
                 const int i = q + 4 * s;
@@ -261,6 +267,10 @@ __device__ __forceinline__ void wg_sweep(const MGI_GLOBAL_AS T* A, int ld, int n
             }
         }
         __syncthreads();
+        // the first tile was loaded during the solve; with it waited for here
+        // the loop's own waits leave the next tile's loads in flight (in the
+        // loop, the wait for either would be for both)
+        __builtin_amdgcn_s_waitcnt(0x0F70);                    // vmcnt(0)
         for (int ti = w; ti < tiles; ti += W) {
             const int row = r0 + 16 * ti + lr;
             const bool rin = row < r1;
