@@ -71,7 +71,10 @@ size_t getrs_generic_bytes(int n, int elem);
 template <typename T>
 magma_int_t getrs_generic_launch_t(int trans, const RsSizes& sz, int max_nrhs, T** dA_array, int** ipiv_array,
                                    T** dB_array, int batch, hipStream_t stream);
-// getrs_wg.hip: one workgroup per system and 32 right-hand sides.
+// getrs_wg.hip: one workgroup per system and 32 right-hand sides, which stay
+// in LDS through both sweeps while they fit in this (several workgroups per
+// CU), and in global memory above it.
+constexpr size_t kGetrsRhsLds = 36 * 1024;
 template <typename T>
 magma_int_t getrs_wg_launch(int trans, const RsSizes& sz, int max_nrhs, T** dA_array, int** ipiv_array, T** dB_array,
                             int batch, hipStream_t stream);

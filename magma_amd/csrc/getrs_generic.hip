@@ -1,6 +1,6 @@
 // Batched triangular solve with LU factors: the choice of kernel, and the
-// kernel for up to four right-hand sides (FP64 or FP32, fixed or per-matrix
-// sizes). Everything else goes to getrs_wg.hip.
+// kernels for up to four right-hand sides at a time (FP64 or FP32, fixed or
+// per-matrix sizes). Everything else goes to getrs_wg.hip.
 #include "magma_internal.h"
 #include "lu_device.h"
 #include "getrf_kernels.h"
@@ -176,6 +176,131 @@ static magma_int_t getrs_wave_launch(const RsSizes& sz, int max_nrhs, T** dA_arr
     return MAGMA_SUCCESS;
 }
 
+// ---------------------------------------------------------------------------
+// Trans with up to four right-hand sides: one workgroup per system, the
+// right-hand sides in LDS, blocks of 64 rows. Wave w solves the block's
+// triangle for right-hand side w (lane l holds row l of the triangle in
+// registers, the solved entry of each step reaches the others by a lane read);
+// then every thread applies the block to the rows left, one row each, with 32
+// of its contiguous factor entries in flight. Bound: the chain of blocks in
+// few systems, HBM in many. Three workgroups per CU (147 registers in FP64):
+// without the bound two, and 768 systems of 256 rows take 1.4 times as long.
+// (The reason to keep it beside the workgroup's sweeps stands at the choice.)
+// ---------------------------------------------------------------------------
+constexpr int kFewRhs = 4;
+
+template <typename T, bool BACK, bool UNIT>
+__device__ __forceinline__ void few_sweep(const MGI_GLOBAL_AS T* __restrict__ A, int ld, int n, T* sB, int nr)
+{
+    const int tid = threadIdx.x, l = tid % kWave, w = tid / kWave;
+    for (int done = 0; done < n; done += kWave) {
+        const int kb = BACK ? max(0, n - done - kWave) : done;
+        const int nb = min(kWave, n - done);
+        if (w < nr) {
+            const int r = kb + l;
+            const bool in = l < nb;
+            T f[kWave];
+            auto Fr = A + kb + (size_t)r * ld;
+#pragma unroll
+            for (int j = 0; j < kWave; ++j) f[j] = (in && (BACK ? j > l && j < nb : j < l)) ? Fr[j] : T(0);
+            const T rd = (!UNIT && in) ? T(1) / A[r + (size_t)r * ld] : T(1);
+            T x = in ? sB[r + w * n] : T(0);
+#pragma unroll
+            for (int jj = 0; jj < kWave; ++jj) {
+                const int j = BACK ? kWave - 1 - jj : jj;
+                if (j < nb) {
+                    T xj = readlane_t(x, j);
+                    if constexpr (!UNIT) {
+                        xj *= readlane_t(rd, j);
+                        if (l == j) x = xj;
+                    }
+                    if (BACK ? l < j : l > j) x = fma(-f[j], xj, x);
+                }
+            }
+            if (in) sB[r + w * n] = x;
+        }
+        __syncthreads();
+        // the rows left exist only beside a full block
+        const int i0 = BACK ? 0 : kb + kWave, i1 = BACK ? kb : n;
+        for (int i = i0 + tid; i < i1; i += kRsThreads) {
+            T acc[kFewRhs];
+#pragma unroll
+            for (int c = 0; c < kFewRhs; ++c) acc[c] = sB[i + c * n];
+            auto Fi = A + kb + (size_t)i * ld;
+            constexpr int CH = 32;
+            for (int j0 = 0; j0 < kWave; j0 += CH) {
+                T f[CH];
+#pragma unroll
+                for (int u = 0; u < CH; ++u) f[u] = Fi[BACK ? kWave - 1 - (j0 + u) : j0 + u];
+#pragma unroll
+                for (int u = 0; u < CH; ++u) {
+                    const int j = BACK ? kWave - 1 - (j0 + u) : j0 + u;
+#pragma unroll
+                    for (int c = 0; c < kFewRhs; ++c) acc[c] = fma(-f[u], sB[kb + j + c * n], acc[c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < kFewRhs; ++c)
+                if (c < nr) sB[i + c * n] = acc[c];
+        }
+        __syncthreads();
+    }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(kRsThreads, sizeof(T) == 8 ? 3 : 4)
+getrs_few_kernel(RsSizes sz, T** __restrict__ dA_array, int** __restrict__ ipiv_array, T** __restrict__ dB_array)
+{
+    extern __shared__ __align__(16) unsigned char rf_raw[];
+    const int b = sz.map ? sz.map[blockIdx.x] : blockIdx.x;
+    int n, nrhs, ldda, lddb;
+    sz.get(b, n, nrhs, ldda, lddb);
+    if (n <= 0 || nrhs <= 0) return;
+    const int nr = min(nrhs, kFewRhs);
+    const int tid = threadIdx.x;
+    T* sB = reinterpret_cast<T*>(rf_raw);                     // n x kFewRhs, the unused columns zero
+    int* perm = reinterpret_cast<int*>(rf_raw + (size_t)sz.max_n * kFewRhs * sizeof(T));
+    int* spiv = perm + sz.max_n;
+    auto A = gptr(dA_array[b]);
+    auto B = gptr(dB_array[b]);
+    auto ipiv = gptr(ipiv_array ? ipiv_array[b] : nullptr);   // null: factors without pivoting
+    // (P^T B)(i,:) = B(perm[i],:): each row is traced back through the
+    // interchanges, last to first; one outside [k, n) is none
+    for (int i = tid; i < n; i += kRsThreads) {
+        const int p = ipiv ? ipiv[i] - 1 : i;
+        spiv[i] = (p > i && p < n) ? p : i;
+#pragma unroll
+        for (int c = 0; c < kFewRhs; ++c) sB[i + c * n] = c < nr ? B[i + (size_t)c * lddb] : T(0);
+    }
+    __syncthreads();
+    for (int r = tid; r < n; r += kRsThreads) {
+        int src = r;
+        for (int k = n - 1; k >= 0; --k) {
+            const int p = spiv[k];
+            src = (src == k) ? p : (src == p ? k : src);
+        }
+        perm[r] = src;
+    }
+    few_sweep<T, false, false>(A, ldda, n, sB, nr);           // U^T
+    few_sweep<T, true, true>(A, ldda, n, sB, nr);             // L^T
+    for (int i = tid; i < n; i += kRsThreads)
+#pragma unroll
+        for (int c = 0; c < kFewRhs; ++c)
+            if (c < nr) B[perm[i] + (size_t)c * lddb] = sB[i + c * n];
+}
+
+template <typename T>
+static magma_int_t getrs_few_launch(const RsSizes& sz, T** dA_array, int** ipiv_array, T** dB_array, int batch,
+                                    hipStream_t stream)
+{
+    const size_t lds = (size_t)sz.max_n * (kFewRhs * sizeof(T) + 2 * sizeof(int));
+    MGI_HIP_CHECK(hipFuncSetAttribute((const void*)getrs_few_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      (int)lds));
+    getrs_few_kernel<T><<<batch, kRsThreads, lds, stream>>>(sz, dA_array, ipiv_array, dB_array);
+    MGI_LAUNCH_CHECK();
+    return MAGMA_SUCCESS;
+}
+
 // The largest order the solve accepts keeps a system's pivots and eight
 // right-hand sides within a workgroup's LDS.
 size_t getrs_generic_bytes(int n, int elem) { return (size_t)n * 8 * elem + 2 * (size_t)n * sizeof(int); }
@@ -187,24 +312,42 @@ magma_int_t getrs_generic_launch_t(int trans, const RsSizes& sz, int max_nrhs, T
 {
     if (batch <= 0 || max_nrhs <= 0) return MAGMA_SUCCESS;
     if (getrs_generic_bytes(sz.max_n, sizeof(T)) > max_dynamic_lds()) return MAGMA_ERR_NOT_SUPPORTED;
-    // up to four right-hand sides of many systems of up to 256 rows read the
-    // factors once in one wave, without barriers (FP64 us, wave against
-    // workgroup: 2,000 x 256^2 r1 276 / 379, r4 320 / 382; 20,000 x 16^2 r2 85 /
-    // 222; 8,192 x 64^2 r1 134 / 212; 5,000 x 100^2 r4 219 / 284); with more, or
-    // above 256 rows, the workgroup's MFMA sweeps win (2,000 x 256^2 r16 935 /
-    // 486, 5,000 x 100^2 r5 361 / 286). Up to four systems per CU the wave's
-    // chain of columns is what counts, and the workgroup's chain of blocks is
-    // shorter (64 x 256^2 r1 174 / 106, r4 221 / 106; 1,024 x 256^2 r1 231 / 199;
-    // 1,024 x 64^2 r4 56 / 38; even at 16 rows). FP32 batches, whose waves
-    // stream half the bytes, stay with the wave at every size (8,192 x 64^2 r1
-    // 80 / 89), and so do mapped buckets, beside which other buckets run.
-    const bool few = sizeof(T) == 8 && sz.map == nullptr && batch <= kFewSystems;
-    if (trans == 0 && sz.max_n <= 256 && max_nrhs <= kWaveCols && !few) {
-        if (sz.max_n <= 64) return getrs_wave_launch<T, 1>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
-        if (sz.max_n <= 128) return getrs_wave_launch<T, 2>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
+    const bool f64 = sizeof(T) == 8;
+    const int n = sz.max_n;
+    if (trans != 0) {
+        // The workgroup's sweeps work on 16 right-hand sides whatever their
+        // number; the row-per-thread kernel is ahead (us, workgroup / few) in
+        // FP64 with one or two of them in systems of a few blocks that the chip
+        // holds all at once (1 x 64^2 r1 43 / 36, 512 x 128^2 r1 72 / 59; 1,024 x
+        // 64^2 r1 49 / 58; from 160 rows on the two are level), and with up to
+        // four that do not stay in the workgroup's LDS (64 x 2,000^2 r4 2975 /
+        // 2262); in FP32, where its contiguous loads count, with one or two from
+        // 193 rows on (3,000 x 512^2 r2 1355 / 1020; 1,100 x 200^2 r1 133 / 136;
+        // 8,192 x 128^2 r1 242 / 292), with up to four from 481 (64 x 1,000^2 r4
+        // 635 / 513; 3,000 x 200^2 r4 263 / 404).
+        const bool few = f64 ? (max_nrhs <= 2 && n > 32 && n <= 128 && batch <= 768) ||
+                                   (size_t)n * max_nrhs * sizeof(T) > kGetrsRhsLds
+                             : max_nrhs <= 2 ? n > 192 : n > 480;
+        if (max_nrhs <= kFewRhs && few) return getrs_few_launch<T>(sz, dA_array, ipiv_array, dB_array, batch, stream);
+        return getrs_wg_launch<T>(trans, sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
+    }
+    // Up to four right-hand sides of many systems of up to 256 rows read the
+    // factors once in one wave, without barriers (us, wave / workgroup: 20,000 x
+    // 16^2 r2 92 / 124, 8,192 x 33^2 r1 79 / 114, 8,192 x 64^2 r1 135 / 135; above
+    // that the workgroup has overtaken it, 8,192 x 128^2 r4 426 / 312, so the
+    // line could come down). Up to four FP64 systems per CU the wave's chain of
+    // columns is what counts, and the workgroup's chain of blocks is shorter
+    // (64 x 256^2 r4 231 / 95; 1,024 x 256^2 r1 234 / 152); mapped buckets, beside
+    // which other buckets run, stay with the wave. With more right-hand sides
+    // the workgroup wins (8,192 x 128^2 r5 705 / 313, FP32 3,000 x 256^2 r5 501 /
+    // 270).
+    const bool few = f64 && sz.map == nullptr && batch <= kFewSystems;
+    if (n <= 256 && max_nrhs <= kWaveCols && !few) {
+        if (n <= 64) return getrs_wave_launch<T, 1>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
+        if (n <= 128) return getrs_wave_launch<T, 2>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
         return getrs_wave_launch<T, 4>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
     }
-    return getrs_wg_launch<T>(trans, sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
+    return getrs_wg_launch<T>(0, sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
 }
 
 template magma_int_t getrs_generic_launch_t<double>(int, const RsSizes&, int, double**, int**, double**, int,

@@ -24,9 +24,6 @@
 
 namespace mgi {
 
-// Right-hand sides are kept in LDS through both sweeps while they fit in this
-// (several workgroups per CU); above it they stay in global memory.
-constexpr size_t kRhsLds = 36 * 1024;
 constexpr int kMaxRhs = 32;      // right-hand sides per workgroup (16 if the batch has no more)
 constexpr int kPermCols = 4;     // right-hand sides permuted at a time in global memory
 
@@ -144,10 +141,10 @@ static magma_int_t launch_nth(const RsSizes& sz, int max_nrhs, T** dA_array, int
     const size_t rhs = (size_t)(sz.max_n | 1) * (max_nrhs < kMaxRhs ? max_nrhs : kMaxRhs) * sizeof(T);
     const size_t gl = perm + (size_t)sz.max_n * kPermCols * sizeof(T);
     if (max_nrhs <= 16)
-        return rhs <= kRhsLds
+        return rhs <= kGetrsRhsLds
                    ? launch_one<T, NTH, TRANS, true, 16>(sz, max_nrhs, perm + rhs, dA_array, ipiv_array, dB_array, batch, stream)
                    : launch_one<T, NTH, TRANS, false, 16>(sz, max_nrhs, gl, dA_array, ipiv_array, dB_array, batch, stream);
-    return rhs <= kRhsLds
+    return rhs <= kGetrsRhsLds
                ? launch_one<T, NTH, TRANS, true, kMaxRhs>(sz, max_nrhs, perm + rhs, dA_array, ipiv_array, dB_array, batch, stream)
                : launch_one<T, NTH, TRANS, false, kMaxRhs>(sz, max_nrhs, gl, dA_array, ipiv_array, dB_array, batch, stream);
 }

@@ -1,6 +1,7 @@
-"""Forms of the batched LU kernels that need large batches to be dispatched,
-run on a few systems through the entries of forms.cpp under the CPU emulation
-with AddressSanitizer (exact-size buffers), against the oracle. One scenario
+"""Forms of the batched LU and solve kernels that scenarios.py does not reach
+(those that need large batches through the entries of forms.cpp), run on a few
+systems under the CPU emulation with AddressSanitizer (exact-size buffers),
+against the oracle. One scenario
 per argument; exits non-zero on the first failure.
 
 Run as scenarios.py (ASan runtime preloaded):
@@ -16,8 +17,9 @@ sys.path.insert(0, str(Path(__file__).resolve().parents[2]))
 
 import oracle  # noqa: E402
 from lu_inputs import dominant_with_zeros, getf2_nopiv, zero_columns_with_nan  # noqa: E402
-from scenarios import FAILURES, LIB, Buf, check, i32, ptr_array, vp  # noqa: E402
+from scenarios import FAILURES, LIB, Buf, check, i32, ptr_array, queue, vp  # noqa: E402
 
+QUEUE = queue()
 LU_FWD_TOL = 1e3 * np.finfo(np.float64).eps
 
 LIB.emu_lu_wave_d.argtypes = [i32, i32, i32, vp, vp, vp, vp, vp, vp, vp, i32, i32, i32]
@@ -63,7 +65,73 @@ def zero_pivot():
         check(info[0] == info_ref and err < LU_FWD_TOL, f"no pivoting {m}x{n}: info {info[0]} {info_ref}, error {err:.1e}")
 
 
-SCENARIOS = {"zero_pivot": zero_pivot}
+def run_getrs(prec, n, nrhs, trans, batch=2, pad=0):
+    """Solve with the oracle's factors of uniform systems; the backward error
+    (FP32: of the system that the rounded factors multiply out to)."""
+    rng = np.random.default_rng(n * 5 + nrhs)
+    dt = np.float64 if prec == "d" else np.float32
+    ld = n + pad
+    A, B = rng.uniform(-1, 1, (batch, n, ld)), rng.uniform(-1, 1, (batch, nrhs, ld)).astype(dt)
+    LU, piv, _ = oracle.dgetrf(A, m=n)
+    bA, bB, bP = Buf(LU.astype(dt)), Buf(B), Buf(piv)
+    pA, pB, pP = (ptr_array(b, batch, b.nbytes // batch) for b in (bA, bB, bP))
+    fn = getattr(LIB, f"magma_{prec}getrs_batched")
+    fn.argtypes = [i32, i32, i32, vp, i32, vp, vp, i32, i32, vp]
+    rc = fn(112 if trans else 111, n, nrhs, pA.ptr, ld, pP.ptr, pB.ptr, ld, batch, QUEUE)
+    X, eye = bB.get(), np.arange(n)
+    check(rc == 0 and np.array_equal(X[:, :, n:], B[:, :, n:]), f"{prec}getrs {n} {nrhs} {trans}: rc {rc} or padding")
+    for s in range(batch):
+        M = LU[s].astype(dt).astype(np.float64)[:, :n].T
+        L, U = np.tril(M, -1), np.triu(M)
+        L[eye, eye] = 1.0
+        P = L @ U
+        for j in reversed(range(n)):                       # undo the interchanges: A = P^T L U
+            P[[j, piv[s][j] - 1]] = P[[piv[s][j] - 1, j]]
+        x, b = X[s, :, :n].astype(np.float64).T, B[s, :, :n].astype(np.float64).T
+        r = np.abs(b - (P.T if trans else P) @ x).max() / (n * np.abs(L).sum(1).max() * np.abs(U).sum(1).max() *
+                                                          np.abs(x).max())
+        check(r < 30 * np.finfo(dt).eps, f"{prec}getrs n={n} nrhs={nrhs} trans={trans}: {r:.1e}")
+
+
+def getrs():
+    """The solve kernels at the edges of their blocks, with the right-hand
+    sides in LDS and in global memory (more than 36 KB of them)."""
+    for prec in "ds":
+        for n, nrhs, pad in ((3, 6, 0), (17, 3, 1), (33, 5, 0), (64, 2, 0), (65, 4, 2), (100, 17, 0), (150, 40, 1),
+                             (257, 1, 0), (290, 4, 3), (300, 40, 0)):
+            for trans in (0, 1):
+                run_getrs(prec, n, nrhs, trans, batch=1 if n > 128 else 2, pad=pad)
+
+
+def getrs_vbatched():
+    """Mixed orders and right-hand side counts, empty ones among them, both
+    directions, where the largest order decides the kernel."""
+    rng = np.random.default_rng(8)
+    for ns, rs in (([40, 0, 100, 33, 7], [2, 1, 1, 0, 2]), ([8, 3, 5], [8, 1, 4]), ([130, 64, 20], [5, 17, 1])):
+        A = [rng.uniform(-1, 1, (1, max(n, 1), max(n, 1))) for n in ns]
+        F = [oracle.dgetrf(a) for a in A]
+        for trans in (0, 1):
+            B = [rng.uniform(-1, 1, (1, max(r, 1), max(n, 1))) for n, r in zip(ns, rs)]
+            bA, bP, bB = [Buf(f[0]) for f in F], [Buf(f[1]) for f in F], [Buf(b) for b in B]
+            pA, pP, pB = (Buf(np.array([x.ptr for x in y], np.uint64)) for y in (bA, bP, bB))
+            dn, dr, ld = Buf(np.array(ns, np.int32)), Buf(np.array(rs, np.int32)), Buf(np.maximum(ns, 1).astype(np.int32))
+            fn = LIB.magma_dgetrs_vbatched
+            fn.argtypes = [i32, vp, vp, i32, i32, vp, vp, vp, vp, vp, i32, vp]
+            rc = fn(112 if trans else 111, dn.ptr, dr.ptr, max(ns), max(rs), pA.ptr, ld.ptr, pP.ptr, pB.ptr, ld.ptr,
+                    len(ns), QUEUE)
+            check(rc == 0, f"dgetrs_vbatched {ns} rc {rc}")
+            for n, r, f, b, x in zip(ns, rs, F, B, bB):
+                X = x.get()
+                if n == 0 or r == 0:
+                    check(np.array_equal(X, b), f"dgetrs_vbatched n={n} nrhs={r}: touched")
+                    continue
+                ref = oracle.dgetrs(trans, f[0], f[1], b)
+                # the oracle solves with the same factors: both errors are of the size n eps times the growth of
+                # the triangles, which uniform factors of these orders keep below 1e8
+                check(np.abs(X - ref).max() <= 1e-7 * np.abs(ref).max(), f"dgetrs_vbatched n={n} nrhs={r} trans={trans}")
+
+
+SCENARIOS = {"zero_pivot": zero_pivot, "getrs": getrs, "getrs_vbatched": getrs_vbatched}
 
 if __name__ == "__main__":
     for name in sys.argv[1:]:

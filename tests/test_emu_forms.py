@@ -1,5 +1,5 @@
-"""Forms of the batched LU kernels that only large batches reach, under the
-CPU emulation with ASan on a few systems, against the oracle."""
+"""Forms of the batched LU and solve kernels that the larger scenarios do not
+reach, under the CPU emulation with ASan on a few systems, against the oracle."""
 import os
 import subprocess
 import sys
@@ -14,7 +14,7 @@ import build_emu  # noqa: E402
 
 
 @pytest.mark.timeout(900)
-@pytest.mark.parametrize("scenario", ["zero_pivot"])
+@pytest.mark.parametrize("scenario", ["zero_pivot", "getrs", "getrs_vbatched"])
 def test_form_under_asan(scenario):
     cxx = build_emu.clang()
     if cxx is None or build_emu.asan_runtime(cxx) is None:
