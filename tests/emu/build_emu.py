@@ -108,6 +108,7 @@ def _shvar(m: re.Match) -> str:
 
 def transform(src: Path, dst: Path) -> list[Path]:
     dst.mkdir(parents=True, exist_ok=True)
+    _SHV_ID[0] = 0                         # the same ids in every call, so that unchanged sources keep their objects
     cpps = []
     for f in sorted(src.glob("*.hip")) + sorted(src.glob("*.h")):
         s = f.read_text()
