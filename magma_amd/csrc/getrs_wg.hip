@@ -25,6 +25,7 @@
 namespace mgi {
 
 constexpr int kMaxRhs = 32;      // right-hand sides per workgroup (16 if the batch has no more)
+constexpr long kOneStrip = 1024; // one-wave workgroups on one wave per SIMD
 constexpr int kPermCols = 4;     // right-hand sides permuted at a time in global memory
 
 template <typename T, int NTH, bool TRANS, bool INLDS, int MAXR>
@@ -138,9 +139,14 @@ static magma_int_t launch_nth(const RsSizes& sz, int max_nrhs, T** dA_array, int
                               hipStream_t stream)
 {
     const size_t perm = (size_t)sz.max_n * 2 * sizeof(int);
-    const size_t rhs = (size_t)(sz.max_n | 1) * (max_nrhs < kMaxRhs ? max_nrhs : kMaxRhs) * sizeof(T);
+    // one wave solves its strips of 16 right-hand sides one after the other: a
+    // workgroup takes one strip while the strips all run at once (us, two strips
+    // / one: 64 x 64^2 r32 60 / 47, 512 x 64^2 r32 64 / 52; 1,024 x 64^2 r32 69 / 80)
+    const bool one = max_nrhs <= 16 || (NTH == kWave && (long)batch * ceildiv(max_nrhs, 16) <= kOneStrip);
+    const int cols = one ? 16 : kMaxRhs;
+    const size_t rhs = (size_t)(sz.max_n | 1) * (max_nrhs < cols ? max_nrhs : cols) * sizeof(T);
     const size_t gl = perm + (size_t)sz.max_n * kPermCols * sizeof(T);
-    if (max_nrhs <= 16)
+    if (one)
         return rhs <= kGetrsRhsLds
                    ? launch_one<T, NTH, TRANS, true, 16>(sz, max_nrhs, perm + rhs, dA_array, ipiv_array, dB_array, batch, stream)
                    : launch_one<T, NTH, TRANS, false, 16>(sz, max_nrhs, gl, dA_array, ipiv_array, dB_array, batch, stream);
