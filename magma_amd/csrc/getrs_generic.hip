@@ -340,9 +340,14 @@ magma_int_t getrs_generic_launch_t(int trans, const RsSizes& sz, int max_nrhs, T
     // (64 x 256^2 r4 231 / 95; 1,024 x 256^2 r1 234 / 152); mapped buckets, beside
     // which other buckets run, stay with the wave. With more right-hand sides
     // the workgroup wins (8,192 x 128^2 r5 705 / 313, FP32 3,000 x 256^2 r5 501 /
-    // 270).
+    // 270), except in systems so small that a wave's work on them is a few
+    // columns (20,000 x 4^2 r5 75 / 108, 20,000 x 8^2 r8 110 / 116, r9 144 / 123;
+    // with more right-hand sides while the waves nearly all run at once: 64 x
+    // 4^2 r64 29 / 33, 64 x 8^2 r32 31 / 33, 2,000 x 8^2 r17 49 / 42).
+    const long waves = (long)batch * ceildiv(max_nrhs, kWaveCols);
+    const bool tiny = n <= 8 && (n * max_nrhs <= 64 || n * waves <= 40960);
     const bool few = f64 && sz.map == nullptr && batch <= kFewSystems;
-    if (n <= 256 && max_nrhs <= kWaveCols && !few) {
+    if (n <= 256 && (tiny || (max_nrhs <= kWaveCols && !few))) {
         if (n <= 64) return getrs_wave_launch<T, 1>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
         if (n <= 128) return getrs_wave_launch<T, 2>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);
         return getrs_wave_launch<T, 4>(sz, max_nrhs, dA_array, ipiv_array, dB_array, batch, stream);

@@ -11,8 +11,10 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 TRANS = 112
-CASES = [(TRANS, n, r, b) for n, r, b in ((32, 2, 9), (33, 1, 768), (33, 2, 769), (128, 2, 30), (129, 2, 30), (64, 3, 30),
-                                          (193, 2, 6), (192, 1, 6), (480, 3, 3), (481, 4, 3), (1536, 3, 3), (1537, 3, 3),
+CASES = [(111, n, r, b) for n, r, b in ((1, 64, 3), (8, 8, 5000), (8, 9, 1706), (8, 9, 1707), (9, 5, 30), (4, 40, 30),
+                                        (16, 17, 512), (16, 17, 513), (33, 40, 3), (64, 33, 30), (65, 33, 3))]
+CASES += [(TRANS, n, r, b) for n, r, b in ((32, 2, 9), (33, 1, 768), (33, 2, 769), (128, 2, 30), (129, 2, 30), (64, 3, 30),
+                                           (193, 2, 6), (192, 1, 6), (480, 3, 3), (481, 4, 3), (1536, 3, 3), (1537, 3, 3),
                                            (1537, 4, 3))]
 
 
