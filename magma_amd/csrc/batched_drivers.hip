@@ -13,7 +13,7 @@ namespace mgi {
 magma_int_t getrf_batched_async(int m, int n, double** dA_array, int ldda, int** ipiv_array,
                                 int* info_array, int batch, hipStream_t stream)
 {
-    if (m == n && getrf_tile_supported(n) && !getrf_wg_over_tile(n, batch))
+    if (m == n && getrf_tile_supported(n) && !getrf_wg_over_tile(n, batch, false))
         return getrf_tile_launch(n, dA_array, ldda, ipiv_array, info_array, batch, stream);
     if (getrf_wg_preferred(m, n, batch)) {
         SizeArgs sz{m, n, ldda, nullptr, nullptr, nullptr, nullptr};
@@ -118,7 +118,7 @@ magma_int_t magma_dgesv_batched(magma_int_t n, magma_int_t nrhs, double** dA_arr
     if (n == 0 || nrhs == 0 || batchCount == 0) return 0;
     if (queue == nullptr) return MAGMA_ERR_NOT_INITIALIZED;
     hipSetDevice(queue->device);
-    if (mgi::gesv_tile_supported(n, nrhs) && !mgi::getrf_wg_over_tile(n, batchCount))
+    if (mgi::gesv_tile_supported(n, nrhs) && !mgi::getrf_wg_over_tile(n, batchCount, true))
         return mgi::gesv_tile_launch(n, nrhs, dA_array, ldda, dipiv_array, dinfo_array, dB_array, lddb,
                                      batchCount, queue->stream);
     if (mgi::getrf_wg_preferred(n, n, batchCount) && nrhs <= 16) {

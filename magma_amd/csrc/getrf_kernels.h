@@ -108,8 +108,9 @@ bool getrf_wg_supported(int max_m);
 // Whether the one-workgroup kernel is the faster choice for a batch of m x n
 // systems (the rule's reasons are at its definition).
 bool getrf_wg_preferred(int max_m, int max_n, int batch);
-// The same against the register-tile kernel, for square systems up to 128.
-bool getrf_wg_over_tile(int max_n, int batch);
+// The same against the register-tile kernel, for square systems up to 128,
+// with the solve of the right-hand sides or without.
+bool getrf_wg_over_tile(int max_n, int batch, bool solve);
 magma_int_t getrf_wg_launch(const SizeArgs& sz, int max_m, double** dA_array, int** ipiv_array, int* info_array,
                             const WgRhs<double>& rhs, int batch, hipStream_t stream);
 magma_int_t sgetrf_wg_launch(int mode, const SizeArgs& sz, int max_m, float** dA_array, int** ipiv_array,

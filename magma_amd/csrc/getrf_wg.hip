@@ -529,7 +529,15 @@ bool getrf_wg_preferred(int max_m, int max_n, int batch)
 // that fit here win above 64 rows. Measured (gesv, FP64, us, tile against
 // this): 1,024 x 100^2 255 / 267, 2,048 x 100^2 478 / 371, 8,192 x 100^2 1781
 // / 1384, 20,000 x 128^2 5463 / 4560; at 64 rows 8,192 systems 508 / 588.
-bool getrf_wg_over_tile(int max_n, int batch) { return max_n > 64 && batch >= 1536; }
+// Without right-hand sides the tile fits three systems of up to 80 rows per CU,
+// all of the time of 80, while here the time grows with the rows: from 69 to 80
+// the tile wins (getrf, 1,536 x 80^2 151 / 176, 2,304 x 72^2 209 / 251, 10,000 x
+// 80^2 743 / 879; 10,000 x 72^2 764 / 805 but 4,000 x 72^2 345 / 323; 4,000 x
+// 65^2 344 / 295, 4,000 x 81^2 496 / 408).
+bool getrf_wg_over_tile(int max_n, int batch, bool solve)
+{
+    return max_n > 64 && batch >= 1536 && (solve || max_n <= 68 || max_n > 80);
+}
 
 template <typename T, int MODE>
 static magma_int_t wg_launch(const SizeArgs& sz, int max_m, T** dA_array, int** ipiv_array, int* info_array,

@@ -110,7 +110,7 @@ static bool build_buckets(const int* h_m, const int* h_n, const int* h_nrhs, int
         if (v == kVbWg && !getrf_wg_supported(vb.max_m)) v = kVbAuto;
         if (variant_nb(v) != 0 && !blocked_nb_valid(vb.max_m, variant_nb(v))) v = kVbAuto;
         if (v == kVbAuto)
-            v = tile_ok && !getrf_wg_over_tile(vb.max_n, vb.count) ? kVbTile
+            v = tile_ok && !getrf_wg_over_tile(vb.max_n, vb.count, solve) ? kVbTile
                 : getrf_wg_preferred(vb.max_m, vb.max_n, vb.count) ? kVbWg : kVbBlocked32;
         if (variant_nb(v) != 0 && !blocked_nb_valid(vb.max_m, variant_nb(v))) {
             v = blocked_nb_valid(vb.max_m, 16) ? kVbBlocked16 : kVbBlocked8;

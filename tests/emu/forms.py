@@ -7,6 +7,7 @@ per argument; exits non-zero on the first failure.
 Run as scenarios.py (ASan runtime preloaded):
       python tests/emu/forms.py zero_pivot
 """
+import ctypes
 import sys
 from pathlib import Path
 
@@ -131,7 +132,25 @@ def getrs_vbatched():
                 check(np.abs(X - ref).max() <= 1e-7 * np.abs(ref).max(), f"dgetrs_vbatched n={n} nrhs={r} trans={trans}")
 
 
-SCENARIOS = {"zero_pivot": zero_pivot, "getrs": getrs, "getrs_vbatched": getrs_vbatched}
+def plan_variants():
+    """The kernel that a plan picks for 65..128 rows by itself: the register
+    tile (1) below 1,536 systems and, without right-hand sides, for 69..80
+    rows; one workgroup per system (6) else."""
+    LIB.magma_dgesv_vbatched_plan_create.argtypes = [vp, vp, i32, vp, vp, ctypes.POINTER(vp)]
+    LIB.magma_vbatched_plan_bucket.argtypes = [vp, i32, ctypes.POINTER(i32)]
+    LIB.magma_vbatched_plan_destroy.argtypes = [vp]
+    for n, count, solve, want in ((68, 1536, False, 6), (69, 1536, False, 1), (80, 1536, False, 1), (81, 1536, False, 6),
+                                  (68, 1535, False, 1), (69, 1536, True, 6), (80, 1536, True, 6), (80, 1535, True, 1)):
+        hn, hr = np.full(count, n, np.int32), np.ones(count, np.int32)
+        plan, info = vp(), (i32 * 5)()
+        rc = LIB.magma_dgesv_vbatched_plan_create(hn.ctypes.data, hr.ctypes.data if solve else None, count, None, QUEUE,
+                                                  ctypes.byref(plan))
+        LIB.magma_vbatched_plan_bucket(plan, 0, info)
+        LIB.magma_vbatched_plan_destroy(plan)
+        check(rc == 0 and info[2] == count and info[1] == want, f"plan of {count} x {n}, solve {solve}: variant {info[1]}")
+
+
+SCENARIOS = {"plan_variants": plan_variants, "zero_pivot": zero_pivot, "getrs": getrs, "getrs_vbatched": getrs_vbatched}
 
 if __name__ == "__main__":
     for name in sys.argv[1:]:
