@@ -533,10 +533,12 @@ bool getrf_wg_preferred(int max_m, int max_n, int batch)
 // all of the time of 80, while here the time grows with the rows: from 69 to 80
 // the tile wins (getrf, 1,536 x 80^2 151 / 176, 2,304 x 72^2 209 / 251, 10,000 x
 // 80^2 743 / 879; 10,000 x 72^2 764 / 805 but 4,000 x 72^2 345 / 323; 4,000 x
-// 65^2 344 / 295, 4,000 x 81^2 496 / 408).
+// 65^2 344 / 295, 4,000 x 81^2 496 / 408), but for the batches of up to 76 rows
+// that run at once here and in three rounds there (2,048 x 72^2 197 / 179).
 bool getrf_wg_over_tile(int max_n, int batch, bool solve)
 {
-    return max_n > 64 && batch >= 1536 && (solve || max_n <= 68 || max_n > 80);
+    const bool one_round = max_n <= 76 && batch > 1536 && batch <= 2048;
+    return max_n > 64 && batch >= 1536 && (solve || max_n <= 68 || max_n > 80 || one_round);
 }
 
 template <typename T, int MODE>

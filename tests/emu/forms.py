@@ -134,13 +134,14 @@ def getrs_vbatched():
 
 def plan_variants():
     """The kernel that a plan picks for 65..128 rows by itself: the register
-    tile (1) below 1,536 systems and, without right-hand sides, for 69..80
-    rows; one workgroup per system (6) else."""
+    tile (1) below 1,536 systems and, without right-hand sides, for 69..80 rows
+    (up to 76 but for 1,537..2,048 systems); one workgroup per system (6) else."""
     LIB.magma_dgesv_vbatched_plan_create.argtypes = [vp, vp, i32, vp, vp, ctypes.POINTER(vp)]
     LIB.magma_vbatched_plan_bucket.argtypes = [vp, i32, ctypes.POINTER(i32)]
     LIB.magma_vbatched_plan_destroy.argtypes = [vp]
     for n, count, solve, want in ((68, 1536, False, 6), (69, 1536, False, 1), (80, 1536, False, 1), (81, 1536, False, 6),
-                                  (68, 1535, False, 1), (69, 1536, True, 6), (80, 1536, True, 6), (80, 1535, True, 1)):
+                                  (68, 1535, False, 1), (76, 1537, False, 6), (76, 2048, False, 6),
+                                  (76, 2049, False, 1), (77, 2048, False, 1), (69, 1536, True, 6), (80, 1536, True, 6), (80, 1535, True, 1)):
         hn, hr = np.full(count, n, np.int32), np.ones(count, np.int32)
         plan, info = vp(), (i32 * 5)()
         rc = LIB.magma_dgesv_vbatched_plan_create(hn.ctypes.data, hr.ctypes.data if solve else None, count, None, QUEUE,
