@@ -15,7 +15,11 @@ magma_int_t getrf_batched_async(int m, int n, double** dA_array, int ldda, int**
 {
     if (m == n && getrf_tile_supported(n) && !getrf_wg_over_tile(n, batch, false))
         return getrf_tile_launch(n, dA_array, ldda, ipiv_array, info_array, batch, stream);
-    if (getrf_wg_preferred(m, n, batch)) {
+    // Wide systems of few rows leave most of the workgroup kernel's lanes and
+    // strips empty: the LDS kernel wins (us, LDS / workgroup: 20,000 x 13 x 20 238 / 274,
+    // 20,000 x 20 x 24 348 / 372, 20 x 40 381 / 379; 24 x 40 452 / 408)
+    const bool short_wide = n > m && m <= 20 && n <= 48;
+    if (!short_wide && getrf_wg_preferred(m, n, batch)) {
         SizeArgs sz{m, n, ldda, nullptr, nullptr, nullptr, nullptr};
         return getrf_wg_launch(sz, m, dA_array, ipiv_array, info_array, WgRhs<double>{}, batch, stream);
     }

@@ -3,6 +3,11 @@ scenarios and the GPU tests."""
 import numpy as np
 
 
+def uniform(rng, batch, m, n):
+    """batch uniform systems, column-major (batch, n, m)."""
+    return rng.uniform(-1, 1, (batch, n, m))
+
+
 def zero_columns_with_nan(rng, n, cols):
     """One uniform system (column-major (1, n, n)), but each of the given
     columns zero except one NaN below the diagonal: its pivot is an exact zero

@@ -49,3 +49,17 @@ def test_zero_pivot_without_pivoting(mb, oracle, m, n, zeros):
     info = mb.dgetrf_nopiv_batched(dA, m=m)
     assert int(info[0]) == info_ref
     assert oracle.lu_forward_error(ref.T[None], dA.cpu().numpy(), m)[0] < LU_FWD_TOL
+
+
+@pytest.mark.parametrize("m,n", [(13, 14), (13, 48), (13, 49), (20, 24), (20, 48), (21, 30)])
+def test_few_wide_rows(mb, oracle, m, n):
+    """Wide systems on both sides of the line to the LDS kernel, 512 of them."""
+    A = lu_inputs.uniform(np.random.default_rng(m * n), 4, m, n)
+    dA = torch.from_numpy(A).cuda().repeat(128, 1, 1)
+    ipiv, info = mb.dgetrf_batched(dA, m=m)
+    LUo, ipo, info_o = oracle.dgetrf(A, m=m)
+    clear = oracle.pivot_margin(A, m) > 1e-10
+    assert (info.cpu().numpy() == 0).all() and (info_o == 0).all()
+    assert np.array_equal(ipiv[-4:].cpu().numpy()[clear], ipo[clear])
+    assert (oracle.lu_forward_error(LUo[clear], dA[-4:].cpu().numpy()[clear], m) < LU_FWD_TOL).all()
+    assert torch.equal(dA, dA[-4:].repeat(128, 1, 1))
