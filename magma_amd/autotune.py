@@ -4,8 +4,8 @@ per system for n <= 512, or the blocked LU with panel width 32, 16 or 8, or
 two 32-wide panels per 64-wide block) by
 timing each valid variant on the bucket's own systems, replayed as a hipGraph.
 Results are cached in a JSON file keyed by device (architecture and CU count)
-and bucket id; `load_variants` reads the cache and tunes only buckets that are
-missing from it.
+and bucket id, with the number of systems that they were timed on; `load_variants`
+reads the cache and tunes only buckets that are missing from it.
 
 The bucket boundaries follow the plan's (magma_amd/csrc/vbatched.hip):
 n <= 128 in steps of 16, then 64 up to 512, 128 up to 1024, 256 up to 2048.
@@ -23,6 +23,10 @@ from .batched import IpivV, VBatch, VbatchedPlan
 
 VARIANT_NAMES = {1: "tile", 2: "blocked nb=32", 3: "blocked nb=16", 4: "blocked nb=8", 5: "blocked 2x32",
                  6: "one workgroup"}
+# From this many systems of 65..128 rows on, one workgroup per system is ahead of
+# the register tile (getrf_wg_over_tile in magma_amd/csrc/getrf_wg.hip).
+WG_OVER_TILE_SYSTEMS = 1536
+TUNE_SYSTEMS = 4096          # systems of a bucket that are timed, at most
 CACHE = Path(os.environ.get("MAGMA_AMD_TUNING", Path(__file__).resolve().parent / "tuning" / "vbatched.json"))
 
 
@@ -73,7 +77,7 @@ def time_plan(plan: VbatchedPlan, A: VBatch, B: VBatch, ipiv: IpivV, info: torch
     return float(np.mean(times[1:]))
 
 
-def tune_buckets(n, nrhs, buckets=None, max_systems: int = 4096, reps: int = 3, seed: int = 1234) -> dict:
+def tune_buckets(n, nrhs, buckets=None, max_systems: int = TUNE_SYSTEMS, reps: int = 3, seed: int = 1234) -> dict:
     """Time every valid variant of each bucket (on up to max_systems of the
     bucket's own systems) and return {bucket: (variant, {variant: seconds})}."""
     n = np.asarray(n, dtype=np.int32)
@@ -110,25 +114,30 @@ def load_variants(n=None, nrhs=None, path: Path = CACHE, tune_missing: bool = Tr
     if path.exists():
         table = json.loads(path.read_text())
     key = device_key()
-    mine = {int(k): int(v["variant"]) for k, v in table.get(key, {}).items()}
-    if n is not None and tune_missing:
-        need = sorted(set(int(b) for b in bucket_of(np.asarray(n)) if b >= 0) - set(mine))
+    cached = table.get(key, {})
+    mine = {int(k): int(v["variant"]) for k, v in cached.items()}
+    if n is None:
+        return mine
+    ids = bucket_of(np.asarray(n))
+    # Tile or one workgroup for 65..128 rows is a matter of how many systems there
+    # are: with few, one system's chain counts, which is shorter on the tile (27
+    # systems of 50..91 rows: 116 us a replay against 161). A choice between the
+    # two holds on its side of the line; an entry without a count stands.
+    for b in range(4, 8):
+        systems, count = cached.get(str(b), {}).get("systems"), int(np.count_nonzero(ids == b))
+        if systems is not None and count and mine[b] in (1, 6):
+            if (systems >= WG_OVER_TILE_SYSTEMS) != (count >= WG_OVER_TILE_SYSTEMS):
+                mine[b] = 6 if count >= WG_OVER_TILE_SYSTEMS else 1
+    if tune_missing:
+        need = sorted(set(int(b) for b in ids if b >= 0) - set(mine))
         if need:
             res = tune_buckets(n, nrhs if nrhs is not None else np.ones(len(n), dtype=np.int32), buckets=need)
             entry = table.setdefault(key, {})
             for b, (v, t) in res.items():
                 entry[str(b)] = {"variant": v, "name": VARIANT_NAMES[v],
+                                 "systems": min(int(np.count_nonzero(ids == b)), TUNE_SYSTEMS),
                                  "seconds": {VARIANT_NAMES[k]: round(s, 6) for k, s in t.items()}}
                 mine[b] = v
             path.parent.mkdir(parents=True, exist_ok=True)
             path.write_text(json.dumps(table, indent=1, sort_keys=True) + "\n")
-    if n is not None:
-        # The cached choice was timed on a full bucket. With fewer systems than
-        # the line that uniform batches have (getrf_wg_over_tile), a bucket of
-        # 65..128 rows is bound by one system's chain, which is shorter on the
-        # tile (27 systems of 50..91 rows: 116 us a replay against 161).
-        ids = bucket_of(np.asarray(n))
-        for b, v in mine.items():
-            if v == 6 and 4 <= b <= 7 and np.count_nonzero(ids == b) < 1536:
-                mine[b] = 1
     return mine
