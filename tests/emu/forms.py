@@ -132,6 +132,24 @@ def getrs_vbatched():
                 check(np.abs(X - ref).max() <= 1e-7 * np.abs(ref).max(), f"dgetrs_vbatched n={n} nrhs={r} trans={trans}")
 
 
+def dense_zero_pivot():
+    """The same on one matrix (magma_dgetrf_gpu, magma_sgetrf_gpu): an exact
+    zero pivot with a NaN below it."""
+    rng = np.random.default_rng(12)
+    for prec, n, cols in (("d", 300, [0, 40, 130]), ("s", 300, [3])):
+        A = zero_columns_with_nan(rng, n, cols)
+        LUo, ipo, info_o = oracle.dgetrf(A)
+        bA = Buf(A[0] if prec == "d" else A[0].astype(np.float32))
+        ipiv, info = (i32 * n)(), i32(-7)
+        fn = getattr(LIB, f"magma_{prec}getrf_gpu")
+        fn.argtypes = [i32, i32, vp, i32, vp, ctypes.POINTER(i32)]
+        rc = fn(n, n, bA.ptr, n, ipiv, ctypes.byref(info))
+        P = np.array(ipiv[:], np.int32)
+        first = int(np.argmax(P != ipo[0])) if not np.array_equal(P, ipo[0]) else -1
+        check(rc >= 0 and info.value == info_o[0], f"dense {prec} zero pivot: rc {rc} info {info.value} {info_o[0]}")
+        check(first < 0, f"dense {prec} zero pivot: pivots differ from step {first}")
+
+
 def plan_variants():
     """The kernel that a plan picks for 65..128 rows by itself: the register
     tile (1) below 1,536 systems and, without right-hand sides, for 69..80 rows
@@ -151,7 +169,7 @@ def plan_variants():
         check(rc == 0 and info[2] == count and info[1] == want, f"plan of {count} x {n}, solve {solve}: variant {info[1]}")
 
 
-SCENARIOS = {"plan_variants": plan_variants, "zero_pivot": zero_pivot, "getrs": getrs, "getrs_vbatched": getrs_vbatched}
+SCENARIOS = {"dense_zero_pivot": dense_zero_pivot, "plan_variants": plan_variants, "zero_pivot": zero_pivot, "getrs": getrs, "getrs_vbatched": getrs_vbatched}
 
 if __name__ == "__main__":
     for name in sys.argv[1:]:

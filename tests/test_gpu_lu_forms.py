@@ -63,3 +63,13 @@ def test_few_wide_rows(mb, oracle, m, n):
     assert np.array_equal(ipiv[-4:].cpu().numpy()[clear], ipo[clear])
     assert (oracle.lu_forward_error(LUo[clear], dA[-4:].cpu().numpy()[clear], m) < LU_FWD_TOL).all()
     assert torch.equal(dA, dA[-4:].repeat(128, 1, 1))
+
+
+def test_dense_zero_pivot_above_a_nan(oracle):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from magma_amd import dense
+    A = lu_inputs.zero_columns_with_nan(np.random.default_rng(12), 300, [0, 40, 130])
+    LUo, ipo, info_o = oracle.dgetrf(A)
+    ipiv, info = dense.getrf_gpu(torch.from_numpy(A[0].copy()).cuda())
+    assert info == info_o[0] and np.array_equal(np.asarray(ipiv), ipo[0])
