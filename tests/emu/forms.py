@@ -17,7 +17,7 @@ sys.path.insert(0, str(Path(__file__).resolve().parent))
 sys.path.insert(0, str(Path(__file__).resolve().parents[2]))
 
 import oracle  # noqa: E402
-from lu_inputs import dominant_with_zeros, getf2_nopiv, zero_columns_with_nan  # noqa: E402
+from lu_inputs import dominant_with_zeros, getf2_nopiv, tied_pairs, zero_columns_with_nan  # noqa: E402
 from scenarios import FAILURES, LIB, Buf, check, i32, ptr_array, queue, vp  # noqa: E402
 
 QUEUE = queue()
@@ -132,6 +132,59 @@ def getrs_vbatched():
                 check(np.abs(X - ref).max() <= 1e-7 * np.abs(ref).max(), f"dgetrs_vbatched n={n} nrhs={r} trans={trans}")
 
 
+def ties():
+    """Candidates that tie, in all bits or in the upper 32: the oracle's pivots."""
+    rng = np.random.default_rng(21)
+    for kernel, sizes in (("wave", (2, 16, 33, 48)), ("wg", (64, 127, 256, 300)), ("wave_f32", (5, 32, 64))):
+        f32 = kernel == "wave_f32"
+        for n in sizes:
+            for _ in range(3):
+                A = tied_pairs(rng, n, 2.0 ** (-20 if f32 else -50))
+                LU, ip, info = run_lu(kernel, A.astype(np.float32) if f32 else A, n)
+                check(info[0] == 0 and np.array_equal(ip, oracle.dgetrf(A)[1]), f"ties {kernel} {n}")
+
+
+def wave():
+    """The FP64 wave kernel with a map, per-matrix orders and leading dimensions
+    (an empty system among them), and fused with up to four right-hand sides."""
+    rng = np.random.default_rng(31)
+    for nch, ns in ((1, [16, 1, 0, 9]), (2, [17, 32, 20, 31]), (3, [48, 33, 47, 40])):
+        lds = [max(n, 1) + k % 3 for k, n in enumerate(ns)]
+        A = [rng.uniform(-1, 1, (1, max(n, 1), ld)) for n, ld in zip(ns, lds)]
+        bA, bP = [Buf(a) for a in A], [Buf(np.zeros(max(n, 1), np.int32)) for n in ns]
+        pA, pP = (Buf(np.array([x.ptr for x in y], np.uint64)) for y in (bA, bP))
+        dn, dl, dm = Buf(np.array(ns, np.int32)), Buf(np.array(lds, np.int32)), Buf(np.array([3, 1, 0, 2], np.int32))
+        info = Buf(np.zeros(4, np.int32))
+        rc = LIB.emu_lu_wave_d(nch, 0, 0, dm.ptr, dn.ptr, dl.ptr, pA.ptr, pP.ptr, info.ptr, None, 0, 0, 4)
+        check(rc == 0 and (info.get() == 0).all(), f"wave {ns}: rc {rc} info {info.get()}")
+        for n, a, b, p in zip(ns, A, bA, bP):
+            if n == 0:
+                check(np.array_equal(b.get(), a), "wave: empty system touched")
+                continue
+            LUo, ipo, _ = oracle.dgetrf(a, m=n)
+            check(np.array_equal(p.get(), ipo[0]), f"wave n={n}: pivots")
+            check(oracle.lu_forward_error(LUo, b.get(), n)[0] < LU_FWD_TOL, f"wave n={n}: factors")
+            check(np.array_equal(b.get()[:, :, n:], a[:, :, n:]), f"wave n={n}: padding touched")
+    for n, nrhs, ld in ((1, 1, 1), (16, 4, 17), (17, 3, 17), (32, 1, 32), (48, 4, 50)):
+        A, B = rng.uniform(-1, 1, (3, n, ld)), rng.uniform(-1, 1, (3, nrhs, ld))
+        bA, bB, bP, bI = Buf(A), Buf(B), Buf(np.zeros((3, n), np.int32)), Buf(np.zeros(3, np.int32))
+        pA, pB, pP = (ptr_array(b, 3, b.nbytes // 3) for b in (bA, bB, bP))
+        rc = LIB.emu_lu_wave_d((n + 15) // 16, n, ld, None, None, None, pA.ptr, pP.ptr, bI.ptr, pB.ptr, nrhs, ld, 3)
+        be = oracle.gesv_backward_error(A, bB.get(), B, n)
+        check(rc == 0 and (be < 30 * np.finfo(np.float64).eps).all(), f"wave gesv n={n} nrhs={nrhs}: {be}")
+
+
+def wide():
+    """Wide systems on the one-workgroup kernel."""
+    rng = np.random.default_rng(41)
+    for m, n in ((20, 50), (33, 40), (64, 100), (130, 145)):
+        A = rng.uniform(-1, 1, (1, n, m))
+        LU, ip, info = run_lu("wg", A, m)
+        LUo, ipo, _ = oracle.dgetrf(A, m=m)
+        check(info[0] == 0 and np.array_equal(ip, ipo), f"wide {m}x{n}: pivots")
+        check(oracle.lu_forward_error(LUo, LU, m)[0] < LU_FWD_TOL, f"wide {m}x{n}: factors")
+
+
 def dense_zero_pivot():
     """The same on one matrix (magma_dgetrf_gpu, magma_sgetrf_gpu): an exact
     zero pivot with a NaN below it."""
@@ -169,7 +222,7 @@ def plan_variants():
         check(rc == 0 and info[2] == count and info[1] == want, f"plan of {count} x {n}, solve {solve}: variant {info[1]}")
 
 
-SCENARIOS = {"dense_zero_pivot": dense_zero_pivot, "plan_variants": plan_variants, "zero_pivot": zero_pivot, "getrs": getrs, "getrs_vbatched": getrs_vbatched}
+SCENARIOS = {f.__name__: f for f in (zero_pivot, dense_zero_pivot, ties, wave, wide, plan_variants, getrs, getrs_vbatched)}
 
 if __name__ == "__main__":
     for name in sys.argv[1:]:

@@ -19,6 +19,21 @@ def zero_columns_with_nan(rng, n, cols):
     return A
 
 
+def tied_pairs(rng, n, ulp):
+    """One system (column-major (1, n, n)) in which every other column has two
+    candidates for its pivot, of magnitude 1 + k ulp, k = 0..3: block upper
+    triangular with 2 x 2 diagonal blocks, its rows permuted. Equal candidates
+    go to the lowest position, which depends on every interchange before, and
+    rounding reaches no candidate of a later pair."""
+    M = np.triu(rng.integers(-3, 4, (n, n)).astype(np.float64), 2)
+    for j in range(0, n - 1, 2):
+        M[j:j + 2, j] = (1 + ulp * rng.integers(0, 4, 2)) * rng.choice([-1.0, 1.0], 2)
+        M[j:j + 2, j + 1] = [0.0, rng.integers(1, 5)]
+    if n % 2:
+        M[n - 1, n - 1] = 2.0
+    return np.ascontiguousarray(M[rng.permutation(n)].T)[None]
+
+
 def dominant_with_zeros(rng, m, n, zeros):
     """m x n with a dominant diagonal, but each of the given rows reaches its
     step unchanged, with a zero on the diagonal."""

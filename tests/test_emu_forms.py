@@ -14,7 +14,8 @@ import build_emu  # noqa: E402
 
 
 @pytest.mark.timeout(900)
-@pytest.mark.parametrize("scenario", ["zero_pivot", "dense_zero_pivot", "plan_variants", "getrs", "getrs_vbatched"])
+@pytest.mark.parametrize("scenario", ["zero_pivot", "dense_zero_pivot", "ties", "wave", "wide", "plan_variants",
+                                      "getrs", "getrs_vbatched"])
 def test_form_under_asan(scenario):
     cxx = build_emu.clang()
     if cxx is None or build_emu.asan_runtime(cxx) is None:

@@ -73,3 +73,20 @@ def test_dense_zero_pivot_above_a_nan(oracle):
     LUo, ipo, info_o = oracle.dgetrf(A)
     ipiv, info = dense.getrf_gpu(torch.from_numpy(A[0].copy()).cuda())
     assert info == info_o[0] and np.array_equal(np.asarray(ipiv), ipo[0])
+
+
+@pytest.mark.parametrize("n,batch", [(2, 2048), (33, 2048), (48, 2048), (48, 2047), (128, 1535), (127, 1536), (128, 1536),
+                                     (256, 3), (301, 3), (512, 3)])
+def test_tied_candidates(mb, oracle, n, batch):
+    A = np.concatenate([lu_inputs.tied_pairs(np.random.default_rng(n + s), n, 2.0 ** -50) for s in range(3)])
+    pick = torch.arange(batch) % 3
+    ipiv, info = mb.dgetrf_batched(torch.from_numpy(A)[pick].cuda())
+    assert (info == 0).all()
+    assert torch.equal(ipiv.cpu(), torch.from_numpy(oracle.dgetrf(A)[1])[pick])
+
+
+@pytest.mark.parametrize("n", [5, 32, 64, 100, 300])
+def test_tied_candidates_f32(mb, oracle, n):
+    A = np.concatenate([lu_inputs.tied_pairs(np.random.default_rng(n + s), n, 2.0 ** -20) for s in range(3)])
+    ipiv, info = mb.sgetrf_batched(torch.from_numpy(A.astype(np.float32)).cuda())
+    assert (info == 0).all() and np.array_equal(ipiv.cpu().numpy(), oracle.dgetrf(A)[1])
