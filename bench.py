@@ -396,6 +396,20 @@ def adjoint_leg(torch, dev, seed, steps=5, batch=8192, n=64, nrhs=8):
     return res
 
 
+def gesv_kernel(n, nrhs, batch):
+    """What magma_dgesv_batched launches (the choices of batched_drivers.hip and getrf_tile.hip)."""
+    from magma_amd.autotune import WG_OVER_TILE_SYSTEMS
+    if nrhs > 16 or n > 512:
+        return "magma_dgesv_batched launch group (getrf + getrs)"
+    if n > 128 or (n > 64 and batch >= WG_OVER_TILE_SYSTEMS):
+        name = f"getrf_wg_kernel<double, {128 if n <= 128 else 256 if n <= 256 else 512}>"
+    elif n <= 48 and nrhs <= 4 and batch >= 2048:
+        name = f"lu_wave_kernel<double, {(n + 15) // 16}, true>"
+    else:
+        name = f"getrf_tile_kernel<{(n + 15) // 16}, true>"
+    return name + " (one fused LU + solve launch per call)"
+
+
 def vbatched_leg(torch, mb, dev, seed, steps=3, batch=50000, nmin=8, nmax=512, rmax=16, spot=48):
     """Variable-size solve: n_i ~ U[nmin, nmax], nrhs_i ~ U[1, rmax], bucketed
     by the plan with the autotuned variant per bucket, captured once as a
@@ -575,8 +589,6 @@ def main():
     ev_avg_s = sum(ev_ms) / len(ev_ms) / 1e3
     achieved = bytes_step / ev_avg_s / 1e9
     workload = f"dgesv_batched {batch} x {n}x{n} FP64, nrhs={nrhs}, ldda={n}"
-    fused = n <= 128 and nrhs <= 16
-    wg = fused and n > 64 and batch >= 1536      # the same line as getrf_wg_over_tile
     roof = {
         "bound": "hbm",
         "achieved": round(achieved, 1),
@@ -584,9 +596,7 @@ def main():
         "unit": "GB/s",
         "frac": round(achieved / HBM_PEAK_GBS, 4),
         "traffic": measured_traffic(workload),
-        "kernel": ("getrf_wg_kernel<double, 128> (one fused LU + solve launch per call)" if wg else
-                   f"getrf_tile_kernel<{(n + 15) // 16}, true> (one fused LU + solve launch per call)" if fused
-                   else "magma_dgesv_batched launch group (getrf + getrs)"),
+        "kernel": gesv_kernel(n, nrhs, batch),
         "event_ms_avg": round(ev_avg_s * 1e3, 4),
         "algorithmic_bytes_per_launch": bytes_step,
         "fp64_tflops": round(flop / ev_avg_s / 1e12, 2),

@@ -95,7 +95,7 @@ magma_int_t sgetrf_blocked_launch(int mode, int m, int n, int ldda, const int* m
                                   int* info_array, int batch, hipStream_t stream);
 
 // getrf_wg.hip: one workgroup per system, at most 512 rows (any columns),
-// with up to 32 right-hand sides carried along and solved (dB_array not null;
+// with up to 16 right-hand sides carried along and solved (dB_array not null;
 // square systems).
 template <typename T>
 struct WgRhs {

@@ -714,7 +714,9 @@ static magma_int_t launch_nt(int nt, const TileArgs& a, double** dA_array, int**
     // eight systems per CU on, up to 48 rows, with at most four of them
     // (FP64 us, tile against wave: getrf 20,000 x 16^2 203 / 108, 2,048 x 48^2
     // 108 / 103; gesv 4,096 x 32^2 r4 129 / 97, 8,192 x 32^2 r8 233 / 211,
-    // 20,000 x 32^2 r16 544 / 679; getrf 8,192 x 64^2 333 / 346)
+    // 20,000 x 32^2 r16 544 / 679; getrf 8,192 x 64^2 333 / 346; kernels alone,
+    // r4: 2,048 x 16^2 27.7 / 26.6, 2,048 x 48^2 84 / 79, 20,000 x 16^2 229 / 161,
+    // 20,000 x 48^2 690 / 607)
     if (nt <= kLuWaveMaxD && batch >= 2048 && (!WITH_B || (a.nrhs_arr == nullptr && a.nrhs <= 4)))
         return lu_wave_launch(nt, a, dA_array, ipiv_array, info_array, dB_array, batch, stream);
     dim3 grid(batch), block(kTileThreads);

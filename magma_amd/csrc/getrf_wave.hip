@@ -14,7 +14,9 @@
 //
 // What bounds it: vector issue (about two lane reads per FP64 entry of each
 // pivot row), with three (FP64) or four waves per SIMD to hide the pivot
-// chain. FP32 8,192 x 64^2: 787 us on the LDS kernel that served it, 364 on
+// chain. At that bound two of the FP64 forms with right-hand sides spill (up to
+// 16 rows 57 registers, 164 bytes of scratch a lane; up to 48 rows 18, 76
+// bytes); the others do not. FP32 8,192 x 64^2: 787 us on the LDS kernel that served it, 364 on
 // one workgroup per system, 228 here (1.2 TB/s).
 //
 // Reference behaviour: magmablas/zgetf2_devicefunc.cuh:218-294 (panel step),

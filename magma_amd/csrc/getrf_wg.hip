@@ -19,9 +19,14 @@
 // the end. With right-hand sides (gesv) B is carried along as more columns
 // on the right and the back substitution follows in the same kernel.
 //
-// What bounds it: at most 128 VGPRs (four waves per SIMD) keeps 16 waves per
-// CU in flight; the panel's dependent chain (about one microsecond per
-// column when alone) is hidden by the other systems of the CU.
+// What bounds it: traffic past the L2 at the copy rate (each block reads and
+// writes the trailing matrix twice). At most 128 VGPRs (four waves per SIMD)
+// keeps 16 waves per CU in flight; the panel's dependent chain (about one
+// microsecond per column when alone) is hidden by the other systems of the CU.
+// The FP64 forms spill 23 registers at that bound (96 bytes of scratch a lane):
+// values kept across a block, and a diagonal block's entries in the back
+// substitution, none in the column steps or the update's MFMA loops. The FP32
+// forms do not spill.
 //
 // Reference behaviour: magmablas/zgetf2_devicefunc.cuh:218-294 (panel step),
 // magmablas/magma_templates.h:44-60 (ties), src/zgetrf_panel_batched.cpp:102-196

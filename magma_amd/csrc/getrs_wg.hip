@@ -11,13 +11,19 @@
 // Bound: HBM on the factors once a CU holds several workgroups; a single
 // system is bound by the chain of its 32-row blocks. Against the sweeps with
 // per-row FMA that it replaced (kernel, us): FP64 1,000 x 384^2 transposed, 16
-// right-hand sides 1219 -> 601 (2.0 TB/s on the factors); FP64 8,192 x 64^2
-// transposed, 8 right-hand sides 562 -> 209; FP32 the same 372 -> 82; FP32
-// 1,000 x 300^2, 8 right-hand sides 6849 -> 157. At small orders the chain of
-// one wave counts: one division per diagonal block instead of one per entry
-// that a thread holds, and eight columns of B in flight instead of one, took
-// whole calls of 8,192 x 64^2 r8 from 265 to 230 us (FP32 111 to 95) and of
-// 20,000 x 16^2 r16 from 377 to 255.
+// right-hand sides 1219 -> 524 (2.3 TB/s on the factors); FP64 8,192 x 64^2
+// transposed, 8 right-hand sides 562 -> 130; FP32 the same 372 -> 71; FP32
+// 1,000 x 300^2, 8 right-hand sides 6849 -> 138.
+//
+// At small orders the chain of one wave counts. What shortened it, in whole
+// calls of FP64 8,192 x 64^2 r8 and 20,000 x 16^2 r16: one division per diagonal
+// block instead of one per entry that a thread holds, and eight columns of B in
+// flight (265 -> 230, 377 -> 255 us); steps past a block's rows skipped, which
+// also ended the spills, and the first tile waited for before the loop over
+// tiles (216 -> 139, 257 -> 138; 1,100 x 512^2 r1 811 -> 594). The forms of more
+// than one wave fit four waves per SIMD without scratch (one of them spills one
+// register); the FP64 one-wave forms take 160..167 + 8 registers, two or three
+// waves per SIMD.
 #include "magma_internal.h"
 #include "getrf_kernels.h"
 #include "wg_lu.h"

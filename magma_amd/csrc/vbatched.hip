@@ -261,9 +261,9 @@ magma_int_t magma_dgetrf_vbatched(magma_int_t* m, magma_int_t* n, double** dA_ar
     return 0;
 }
 
-// include/magma_zvbatched.h:73. No argument checks and no host sync: one
-// blocked launch sequence over the whole batch (sizes stay on the device),
-// sized by the caller's maxima. The workspace holds nothing; a query returns
+// include/magma_zvbatched.h:73. No argument checks and no host sync: the whole
+// batch in the one-workgroup kernel's launch or one blocked launch sequence
+// (sizes stay on the device), chosen and sized by the caller's maxima. The workspace holds nothing; a query returns
 // a minimal size.
 magma_int_t magma_dgetrf_vbatched_max_nocheck_work(magma_int_t* m, magma_int_t* n, magma_int_t max_m,
                                                    magma_int_t max_n, magma_int_t max_minmn, magma_int_t max_mxn,
